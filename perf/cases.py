@@ -700,19 +700,24 @@ def _potential(g, b):
     A = lambda x: g.d0t(g.h1 * g.d0(x))  # noqa: E731
     D = _add(g.nv, g.v0, g.h1) + _add(g.nv, g.v1, g.h1)
     r = g.h0 * b
-    x, start = torch.zeros_like(r), r.norm()
+    x, best, least = torch.zeros_like(r), None, r.norm()
+    start = least
     z = r / D
     p, rz = z, r @ z
     for k in range(20000):
         q = A(p)
         alpha = rz / (p @ q)
         x, r = x + alpha * p, r - alpha * q
-        if k % 100 == 0 and r.norm() < 1e-13 * start:
-            break
+        if k % 10 == 9:
+            size = r.norm()
+            if size < least:
+                best, least = x, size
+            if size < 1e-13 * start or not size < 1e3 * least:
+                break
         z = r / D
         old, rz = rz, r @ z
         p = z + rz / old * p
-    return x
+    return best
 
 
 def _network(g, th, r):
