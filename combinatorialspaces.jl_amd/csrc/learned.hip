@@ -701,16 +701,27 @@ __device__ __forceinline__ void mfma_tile(const unsigned short *rows, int q, int
   }
 }
 
+// A batch of B samples (rows of sample b at b n): the B T tiles in sample
+// order, T = ceil(n / 64) tiles each.
 template <int W>
-__global__ void __launch_bounds__(64) k_inf_layer2w(int n, const int *__restrict__ pcol, const float *__restrict__ pval,
+__global__ void __launch_bounds__(64) k_inf_layer2w(int n, int B, const int *__restrict__ pcol,
+                                                    const float *__restrict__ pval,
                                                     const unsigned short *__restrict__ h1,
                                                     const float *__restrict__ th, unsigned short *__restrict__ h2) {
   __shared__ __align__(16) unsigned short rows[64 * kRowPitch];
   int lane = threadIdx.x;
   int li = lane & 15, lg = lane >> 4;
   const int sub = lane >> 2, part = lane & 3;
+  const int T = (n + 63) / 64;
   int t = dec_ell::xcd_block();
-  if (t >= (n + 63) / 64) return;
+  if (t >= B * T) return;
+  if (B > 1) {
+    int b = t / T;
+    t -= b * T;
+    size_t o = static_cast<size_t>(b) * n * H;
+    h1 += o;
+    h2 += o;
+  }
   short4_t Bw[2][4];
   load_wB(th + OW2, li, lg, Bw);
   float bias0 = th[OB2 + li], bias1 = th[OB2 + 16 + li];
@@ -1166,6 +1177,573 @@ __global__ void k_hp_grad(int n, float scale, const float *__restrict__ eh, cons
   g[o] = scale * (eh[o] - t[o]);
 }
 
+// ---- training: forward and backward of a batch in BF16 ----------------------
+// Rows of P of at most 8 slots (the general kernels above take wider ones).
+// The B samples' rows are cut into 64-row tiles, one wavefront each, dealt to
+// the XCDs in contiguous ranges, so that a sample's rows (2.6 MB of h at 40,962
+// rows) are gathered from one XCD's L2.
+//
+// forward   k_fwd_input -> h1, k_inf_layer2w -> h2, k_fwd_layer3w -> h3
+// backward  k_head_back: dy and the sign mask of h3 per row, the head's sums
+//           k_layer_back<HEAD>: layer 3's weights, dz2
+//           k_layer_back: layer 2's weights, layer 1's weights
+// With q = Pᵀ dz, a layer's gradients are dW = [hᵀ dz; hᵀ q] and
+// dh = dz W_ownᵀ + q W_nbᵀ (P h and dz Wᵀ are never stored): the only rows that
+// are gathered are dz's own 64 bytes, and at the head 8 bytes (dy, mask) from
+// which a neighbour's dz3 is formed again.  q is summed in FP32 and enters the
+// matrix products as the sum of two BF16 values.  Each workgroup adds its
+// tiles' parameter sums in registers and writes one row of `part`
+// (kBackBlocks rows of NP); k_reduce_params adds the rows in double.
+//
+// What bounds them: the h and dz rows read and written (0.46 GB at 16 x 40,962
+// rows, about 90 µs of HBM time) and the gathers' dependent loads.  Measured at
+// that size, loss and gradient of the error loss: 338 µs, against 2,020 µs with
+// one kernel per operation (dg in FP32, two launches per reduction), the
+// gradient as far from its value in 64 bits as before (4.1e-3 of its norm).
+
+constexpr int kBackBlocks = 512;           // at most; a multiple of 8
+constexpr int kBackPitch = 4 * H + 8;      // bf16 per LDS row: [dz | q high | q low | h] plus padding
+
+// x = r / s, P x and the layer-1 rows h1 (the values of k_input).
+template <int W>
+__global__ void __launch_bounds__(TB) k_fwd_input(int n, int B, const int *__restrict__ pcol,
+                                                  const float *__restrict__ pval, const float *__restrict__ r,
+                                                  const float *__restrict__ s, const float *__restrict__ th,
+                                                  float *__restrict__ x, float *__restrict__ px,
+                                                  unsigned short *__restrict__ h1) {
+  const int T = (n + 63) / 64;
+  int lane = threadIdx.x & 63;
+  int t = dec_ell::xcd_block() * kInfWaves + (threadIdx.x >> 6);
+  if (t >= B * T) return;
+  int b = t / T;
+  t -= b * T;
+  size_t o = static_cast<size_t>(b) * n;
+  r += o;
+  x += o;
+  px += o;
+  h1 += o * H;
+  int v = t * 64 + lane, vv = min(v, n - 1);
+  float inv = 1.0f / s[b];
+  int c[W];
+  float pv[W], rc[W];
+#pragma unroll
+  for (int k = 0; k < W; k++) {
+    c[k] = pcol[k * static_cast<size_t>(n) + vv];
+    pv[k] = pval[k * static_cast<size_t>(n) + vv];
+  }
+  float xv = r[vv] * inv;
+#pragma unroll
+  for (int k = 0; k < W; k++) rc[k] = r[c[k] < 0 ? vv : c[k]];
+  float acc = 0.0f;
+#pragma unroll
+  for (int k = 0; k < W; k++) {
+    float tk = pv[k] * (rc[k] * inv);
+    acc = c[k] >= 0 ? acc + tk : acc;
+  }
+  if (v < n) {
+    x[v] = xv;
+    px[v] = acc;
+  }
+  const int sub = lane >> 2, q = lane & 3;
+  float w0[8], w1[8], b1[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    w0[e] = th[OW1 + 8 * q + e];
+    w1[e] = th[OW1 + H + 8 * q + e];
+    b1[e] = th[OB1 + 8 * q + e];
+  }
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    int src = 16 * g + sub;
+    float xg = __shfl(xv, src), ag = __shfl(acc, src);
+    float hh[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      float z = xg * w0[e] + ag * w1[e] + b1[e];
+      hh[e] = z > 0.0f ? z : 0.0f;
+    }
+    int row = t * 64 + src;
+    if (row < n) *reinterpret_cast<uint4 *>(h1 + static_cast<size_t>(row) * H + 8 * q) = pack8(hh);
+  }
+}
+
+// h3 = relu([h2, P h2] W3 + b3) (stored when h3 is given), y = alpha x +
+// h3 wo + bo (stored when y is given), c = (s / D) y (when given), and with
+// the errors e, eps = κ (e / s - y / D) in place of y (the values of
+// k_dense_bf16, k_output and k_err).
+template <int W>
+__global__ void __launch_bounds__(64) k_fwd_layer3w(int n, int B, const int *__restrict__ pcol,
+                                                    const float *__restrict__ pval,
+                                                    const unsigned short *__restrict__ h2,
+                                                    const float *__restrict__ x, const float *__restrict__ th,
+                                                    const float *__restrict__ s, const float *__restrict__ D, float kap,
+                                                    const float *__restrict__ e, unsigned short *__restrict__ h3,
+                                                    float *__restrict__ y, float *__restrict__ c_out) {
+  __shared__ __align__(16) unsigned short rows[64 * kRowPitch];
+  int lane = threadIdx.x;
+  int li = lane & 15, lg = lane >> 4;
+  const int sub = lane >> 2, part = lane & 3;
+  const int T = (n + 63) / 64;
+  int t = dec_ell::xcd_block();
+  if (t >= B * T) return;
+  int b = t / T;
+  t -= b * T;
+  size_t o = static_cast<size_t>(b) * n;
+  h2 += o * H;
+  short4_t Bw[2][4];
+  load_wB(th + OW3, li, lg, Bw);
+  float bias0 = th[OB3 + li], bias1 = th[OB3 + 16 + li];
+  float alpha = th[OAL], bo = th[OBO], sc = s[b];
+  int v = t * 64 + lane;
+  int vv = min(v, n - 1);
+  int c[W];
+  float pv[W];
+  own_slots<W>(n, v, pcol, pval, c, pv);
+  float xv = x[o + vv], dv = D[vv], ev = e ? e[o + vv] : 0.0f;
+  coop_rows_g<W>(n, t, lane, c, pv, h2, rows);
+  wave_sync();
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    float4_t acc[2];
+    mfma_tile(rows, q, li, lg, Bw, acc);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      unsigned short *d = rows + (16 * q + 4 * lg + i) * kRowPitch;
+      float z0 = acc[0][i] + bias0, z1 = acc[1][i] + bias1;
+      d[li] = f2bf(z0 > 0.0f ? z0 : 0.0f);
+      d[16 + li] = f2bf(z1 > 0.0f ? z1 : 0.0f);
+    }
+  }
+  wave_sync();
+  const uint4 *my = reinterpret_cast<const uint4 *>(rows + lane * kRowPitch);
+  float hw = 0.0f;
+#pragma unroll
+  for (int k4 = 0; k4 < 4; k4++) {
+    float f[8];
+    unpack8(my[k4], f);
+#pragma unroll
+    for (int j = 0; j < 8; j++) hw = hw + f[j] * th[OWO + 8 * k4 + j];
+  }
+  float yy = alpha * xv + hw + bo;
+  if (v < n) {
+    if (y) y[o + v] = e ? kap * (ev / sc - yy / dv) : yy;
+    if (c_out) c_out[o + v] = (sc / dv) * yy;
+  }
+  if (!h3) return;
+  h3 += o * H;
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    int r = t * 64 + 16 * g + sub;
+    if (r < n)
+      *reinterpret_cast<uint4 *>(h3 + static_cast<size_t>(r) * H + 8 * part) =
+          *reinterpret_cast<const uint4 *>(rows + (16 * g + sub) * kRowPitch + 8 * part);
+  }
+}
+
+// eh = eps - Pr crs (crs = R eps) in place of eps, and the block partials of Σ eh²
+__global__ void __launch_bounds__(TB) k_prolong_hp(int n, int nc, int width, const int *__restrict__ col,
+                                                   const float *__restrict__ val, const float *__restrict__ crs,
+                                                   float *__restrict__ eps, double *__restrict__ part) {
+  __shared__ double sh[TB];
+  int v = blockIdx.x * blockDim.x + threadIdx.x;
+  int b = blockIdx.y;
+  double sq = 0.0;
+  if (v < n) {
+    size_t o = static_cast<size_t>(b) * n + v;
+    float eh = eps[o] - dec_ell::row<0, float, float>(n, width, v, col, val, crs + static_cast<size_t>(b) * nc);
+    eps[o] = eh;
+    sq = static_cast<double>(eh) * eh;
+  }
+  sh[threadIdx.x] = sq;
+  __syncthreads();
+  for (int w = TB / 2; w > 0; w >>= 1) {
+    if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = sh[0];
+}
+
+// Σ over the workgroup's four waves of 64 x K per-lane values (K at a time in LDS), lane l of wave 0 holding it
+template <int K>
+__device__ __forceinline__ void add_waves(float (&v)[K], float *lds) {
+  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; k++) lds[(w * K + k) * 64 + lane] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    v[k] = 0.0f;
+#pragma unroll
+    for (int q = 0; q < kInfWaves; q++) v[k] = v[k] + lds[(q * K + k) * 64 + lane];
+  }
+}
+
+// The tiles of this wavefront: XCD x (workgroups ≡ x mod 8) takes the x-th
+// contiguous eighth of the `total` tiles, its wavefronts side by side.
+__device__ __forceinline__ void wave_tiles(int total, int &first, int &end, int &step) {
+  int x = blockIdx.x & 7;
+  first = static_cast<int>(static_cast<long long>(total) * x / 8);
+  end = static_cast<int>(static_cast<long long>(total) * (x + 1) / 8);
+  step = (gridDim.x >> 3) * kInfWaves;
+  first += (blockIdx.x >> 3) * kInfWaves + (threadIdx.x >> 6);
+}
+
+// dy = -(Aᵀ dρ) / D (residual loss: a = Aᵀ, g = dρ) or -scale (eh - Rᵀ crs) / D
+// (error loss: a = Rᵀ over nc columns, g = eh); per row (dy, the signs of h3 as
+// 32 bits) for k_layer_back, and the sums Σ dy h3, Σ dy, Σ dy x of wo, bo, alpha.
+template <bool ERR>
+__global__ void __launch_bounds__(TB) k_head_back(int n, int B, int nc, int aw, const int *__restrict__ acol,
+                                                  const float *__restrict__ aval, const float *__restrict__ g,
+                                                  const float *__restrict__ crs, float scale,
+                                                  const float *__restrict__ D, const float *__restrict__ x,
+                                                  const unsigned short *__restrict__ h3, float2 *__restrict__ dm,
+                                                  float *__restrict__ part_out) {
+  __shared__ float red[kInfWaves * 10 * 64];
+  const int lane = threadIdx.x & 63, sub = lane >> 2, part = lane & 3;
+  const int T = (n + 63) / 64;
+  float sums[10];  // Σ dy h3 of the features 8 part .. + 7, then Σ dy and Σ dy x of the lane's rows
+#pragma unroll
+  for (int k = 0; k < 10; k++) sums[k] = 0.0f;
+  int w, wend, step;
+  wave_tiles(B * T, w, wend, step);
+  for (; w < wend; w += step) {
+    int b = w / T, t = w - b * T;
+    size_t o = static_cast<size_t>(b) * n;
+    int v = t * 64 + lane, vv = min(v, n - 1);
+    float a;
+    if constexpr (ERR)
+      a = scale * (g[o + vv] - dec_ell::row<0, float, float>(n, aw, vv, acol, aval, crs + static_cast<size_t>(b) * nc));
+    else
+      a = dec_ell::row<0, float, float>(n, aw, vv, acol, aval, g + o);
+    float dy = v < n ? -a / D[vv] : 0.0f;
+    sums[8] += dy;
+    sums[9] += dy * x[o + vv];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      int r = t * 64 + 16 * q + sub;
+      uint4 hr = *reinterpret_cast<const uint4 *>(h3 + (o + min(r, n - 1)) * H + 8 * part);
+      float d = __shfl(dy, 16 * q + sub);
+      float f[8];
+      unpack8(hr, f);
+      unsigned int m = 0;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        sums[e] += d * f[e];
+        m |= (f[e] > 0.0f ? 1u : 0u) << e;
+      }
+      m <<= 8 * part;
+      m |= __shfl_xor(m, 1);
+      m |= __shfl_xor(m, 2);
+      if (part == 0 && r < n) dm[o + r] = make_float2(d, __uint_as_float(m));
+    }
+  }
+#pragma unroll
+  for (int off = 4; off < 64; off <<= 1)
+#pragma unroll
+    for (int k = 0; k < 8; k++) sums[k] += __shfl_xor(sums[k], off);
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    sums[8] += __shfl_xor(sums[8], off);
+    sums[9] += __shfl_xor(sums[9], off);
+  }
+  add_waves<10>(sums, red);
+  float *out = part_out + static_cast<size_t>(blockIdx.x) * NP;
+  if (threadIdx.x < 4) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) out[OWO + 8 * part + e] = sums[e];
+    if (part == 0) {
+      out[OBO] = sums[8];
+      out[OAL] = sums[9];
+    }
+  }
+}
+
+// four consecutive rows' entries of one LDS column, as an MFMA operand over rows
+__device__ __forceinline__ short4_t lds_col4(const unsigned short *p) {
+  short4_t a;
+  a[0] = static_cast<short>(p[0]);
+  a[1] = static_cast<short>(p[kBackPitch]);
+  a[2] = static_cast<short>(p[2 * kBackPitch]);
+  a[3] = static_cast<short>(p[3 * kBackPitch]);
+  return a;
+}
+
+// One dense layer's backward step.  dz of the layer: HEAD, formed from dm (dy
+// and the sign mask of h3) and wo; else the stored rows dzin.  hb: the rows the
+// layer read.  Weights Wt (64 x 32).  Sums of the layer's dW at ow; of
+// g = dh ⊙ [hb > 0] at ob_below; HEAD: of dz at ob_self, and g is stored in BF16
+// as the dz of the layer below; else: of (x g, P x g) at OW1.
+template <int W, bool HEAD>
+__global__ void __launch_bounds__(TB)
+    k_layer_back(int n, int B, const int *__restrict__ ptcol, const float *__restrict__ ptval,
+                 const unsigned short *__restrict__ dzin, const float2 *__restrict__ dm, const float *__restrict__ wo,
+                 const unsigned short *__restrict__ hb, const float *__restrict__ Wt, unsigned short *__restrict__ dzout,
+                 const float *__restrict__ x, const float *__restrict__ px, float *__restrict__ part_out, int ow,
+                 int ob_below, int ob_self) {
+  __shared__ __align__(16) unsigned short rows_s[kInfWaves][64 * kBackPitch];
+  __shared__ float2 xs_s[HEAD ? 1 : kInfWaves][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int li = lane & 15, lg = lane >> 4, sub = lane >> 2, part = lane & 3;
+  unsigned short *rows = rows_s[wv];
+  const int T = (n + 63) / 64;
+  // Wᵀ as B operands: own rows of W and neighbour rows
+  short4_t Bo[2][2], Bn[2][2];
+#pragma unroll
+  for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        int j = ks * 16 + 4 * lg + i, f = jt * 16 + li;
+        Bo[jt][ks][i] = static_cast<short>(f2bf(Wt[f * H + j]));
+        Bn[jt][ks][i] = static_cast<short>(f2bf(Wt[(H + f) * H + j]));
+      }
+  float wl[8];
+  if constexpr (HEAD) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) wl[e] = wo[8 * part + e];
+  }
+  float4_t aO[2][2], aN[2][2];  // dW tiles: features 16 ft.., columns 16 jt..
+#pragma unroll
+  for (int ft = 0; ft < 2; ft++)
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++) aO[ft][jt] = aN[ft][jt] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float osum[8], bsum[2] = {0.0f, 0.0f}, w1[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int e = 0; e < 8; e++) osum[e] = 0.0f;
+  int wt, wend, step;
+  wave_tiles(B * T, wt, wend, step);
+  for (; wt < wend; wt += step) {
+    int b = wt / T, t = wt - b * T;
+    const size_t o = static_cast<size_t>(b) * n;
+    int c[W];
+    float pv[W];
+    own_slots<W>(n, t * 64 + lane, ptcol, ptval, c, pv);
+    if constexpr (!HEAD) {
+      int vv = min(t * 64 + lane, n - 1);
+      xs_s[wv][lane] = make_float2(x[o + vv], px[o + vv]);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      int r = t * 64 + 16 * g + sub;
+      size_t rr = o + min(r, n - 1);
+      int cg[W];
+      float vg[W];
+#pragma unroll
+      for (int k = 0; k < W; k++) {
+        cg[k] = __shfl(c[k], 16 * g + sub);
+        vg[k] = __shfl(pv[k], 16 * g + sub);
+      }
+      uint4 hr = *reinterpret_cast<const uint4 *>(hb + rr * H + 8 * part);
+      float q[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) q[e] = 0.0f;
+      uint4 own;
+      if constexpr (HEAD) {
+        float2 od = dm[rr], nd[W];
+#pragma unroll
+        for (int k = 0; k < W; k++) nd[k] = dm[o + (cg[k] < 0 ? 0 : cg[k])];
+        auto form = [&](float2 d, bool keep) {
+          unsigned int m = keep ? __float_as_uint(d.y) >> (8 * part) : 0u;
+          float z[8];
+#pragma unroll
+          for (int e = 0; e < 8; e++) z[e] = (m >> e) & 1u ? d.x * wl[e] : 0.0f;
+          return pack8(z);
+        };
+        own = form(od, r < n);
+        float f[8];
+        unpack8(own, f);
+#pragma unroll
+        for (int e = 0; e < 8; e++) osum[e] += f[e];
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+          unpack8(form(nd[k], cg[k] >= 0), f);
+#pragma unroll
+          for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
+        }
+      } else {
+        own = keep_if(*reinterpret_cast<const uint4 *>(dzin + rr * H + 8 * part), r < n);
+        uint4 a[W];
+#pragma unroll
+        for (int k = 0; k < W; k++)
+          a[k] = keep_if(*reinterpret_cast<const uint4 *>(dzin + (o + (cg[k] < 0 ? 0 : cg[k])) * H + 8 * part),
+                         cg[k] >= 0);
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+          float f[8];
+          unpack8(a[k], f);
+#pragma unroll
+          for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
+        }
+      }
+      uint4 hi = pack8(q);
+      float fh[8];
+      unpack8(hi, fh);
+#pragma unroll
+      for (int e = 0; e < 8; e++) q[e] = q[e] - fh[e];
+      unsigned short *d = rows + (16 * g + sub) * kBackPitch + 8 * part;
+      *reinterpret_cast<uint4 *>(d) = own;
+      *reinterpret_cast<uint4 *>(d + H) = hi;
+      *reinterpret_cast<uint4 *>(d + 2 * H) = pack8(q);
+      *reinterpret_cast<uint4 *>(d + 3 * H) = keep_if(hr, r < n);
+    }
+    wave_sync();
+    // dW += hᵀ dz, hᵀ q: four steps of 16 rows
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) {
+      const unsigned short *base = rows + (16 * ks + 4 * lg) * kBackPitch + li;
+      short4_t A[2], Z[2], Q[2], L[2];
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        A[k] = lds_col4(base + 3 * H + 16 * k);
+        Z[k] = lds_col4(base + 16 * k);
+        Q[k] = lds_col4(base + H + 16 * k);
+        L[k] = lds_col4(base + 2 * H + 16 * k);
+      }
+#pragma unroll
+      for (int ft = 0; ft < 2; ft++)
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++) {
+          aO[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], Z[jt], aO[ft][jt], 0, 0, 0);
+          aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], Q[jt], aN[ft][jt], 0, 0, 0);
+          aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], L[jt], aN[ft][jt], 0, 0, 0);
+        }
+    }
+    // dh of 16 rows at a time, masked by the signs of h
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const unsigned short *rp = rows + (16 * g + li) * kBackPitch + 4 * lg;
+      short4_t Z[2] = {lds4(rp), lds4(rp + 16)}, Q[2] = {lds4(rp + H), lds4(rp + H + 16)},
+               L[2] = {lds4(rp + 2 * H), lds4(rp + 2 * H + 16)};
+#pragma unroll
+      for (int jt = 0; jt < 2; jt++) {
+        float4_t a = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+          a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Z[ks], Bo[jt][ks], a, 0, 0, 0);
+          a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(L[ks], Bn[jt][ks], a, 0, 0, 0);
+          a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Q[ks], Bn[jt][ks], a, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          int row = 16 * g + 4 * lg + i;
+          unsigned short *d = rows + row * kBackPitch;
+          // h is zero in rows past the end, so those add nothing
+          float gv = bf2f(d[3 * H + 16 * jt + li]) > 0.0f ? a[i] : 0.0f;
+          bsum[jt] += gv;
+          if constexpr (HEAD) {
+            d[16 * jt + li] = f2bf(gv);
+          } else {
+            float2 xp = xs_s[wv][row];
+            w1[jt] += xp.x * gv;
+            w1[2 + jt] += xp.y * gv;
+          }
+        }
+      }
+    }
+    wave_sync();
+    if constexpr (HEAD) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        int r = t * 64 + 16 * g + sub;
+        if (r < n)
+          *reinterpret_cast<uint4 *>(dzout + (o + r) * H + 8 * part) =
+              *reinterpret_cast<const uint4 *>(rows + (16 * g + sub) * kBackPitch + 8 * part);
+      }
+      wave_sync();
+    }
+  }
+  // the wavefronts' sums into one row of partials
+  float *out = part_out + static_cast<size_t>(blockIdx.x) * NP;
+  float *lds = reinterpret_cast<float *>(rows_s);
+  {
+    float v[32];
+#pragma unroll
+    for (int ft = 0; ft < 2; ft++)
+#pragma unroll
+      for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          v[(ft * 2 + jt) * 4 + i] = aO[ft][jt][i];
+          v[16 + (ft * 2 + jt) * 4 + i] = aN[ft][jt][i];
+        }
+    add_waves<32>(v, lds);
+    if (threadIdx.x < 64) {
+#pragma unroll
+      for (int ft = 0; ft < 2; ft++)
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            int f = 16 * ft + 4 * lg + i, j = 16 * jt + li;
+            out[ow + f * H + j] = v[(ft * 2 + jt) * 4 + i];
+            out[ow + (H + f) * H + j] = v[16 + (ft * 2 + jt) * 4 + i];
+          }
+    }
+  }
+  float v[6] = {bsum[0], bsum[1], w1[0], w1[1], w1[2], w1[3]};
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    v[k] += __shfl_xor(v[k], 16);
+    v[k] += __shfl_xor(v[k], 32);
+  }
+  add_waves<6>(v, lds);
+  if (threadIdx.x < 16) {
+    out[ob_below + li] = v[0];
+    out[ob_below + 16 + li] = v[1];
+    if constexpr (!HEAD) {
+      out[OW1 + li] = v[2];
+      out[OW1 + 16 + li] = v[3];
+      out[OW1 + H + li] = v[4];
+      out[OW1 + H + 16 + li] = v[5];
+    }
+  }
+  if constexpr (HEAD) {
+#pragma unroll
+    for (int off = 4; off < 64; off <<= 1)
+#pragma unroll
+      for (int e = 0; e < 8; e++) osum[e] += __shfl_xor(osum[e], off);
+    add_waves<8>(osum, lds);
+    if (threadIdx.x < 4) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) out[ob_self + 8 * part + e] = osum[e];
+    }
+  }
+}
+
+// grad[j] = Σ_p part[p][j] in double, in a fixed order: 16 wavefronts each add
+// a run of the rows, then the 16 sums in order.  `loss` (workgroup past the
+// columns): scale Σ lpart.
+__global__ void __launch_bounds__(1024) k_reduce_params(int nparts, const float *__restrict__ part,
+                                                        float *__restrict__ grad, int nl,
+                                                        const double *__restrict__ lpart, double scale,
+                                                        double *__restrict__ loss) {
+  __shared__ double sh[16][64];
+  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double acc = 0.0;
+  bool last = blockIdx.x + 1 == gridDim.x;
+  if (last) {
+    for (int p = threadIdx.x; p < nl; p += 1024) acc += lpart[p];
+  } else {
+    int j = min(static_cast<int>(blockIdx.x) * 64 + lane, NP - 1);
+    int per = (nparts + 15) / 16, p1 = min(nparts, (w + 1) * per);
+#pragma unroll 8
+    for (int p = w * per; p < p1; p++) acc += static_cast<double>(part[static_cast<size_t>(p) * NP + j]);
+  }
+  sh[w][lane] = acc;
+  __syncthreads();
+  if (w != 0) return;
+  double t = 0.0;
+  for (int k = 0; k < 16; k++) t += sh[k][lane];
+  if (last) {
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off);
+    if (lane == 0) *loss = t * scale;
+  } else if (static_cast<int>(blockIdx.x) * 64 + lane < NP) {
+    grad[blockIdx.x * 64 + lane] = static_cast<float>(t);
+  }
+}
+
 // dy = -(Aᵀ dρ) / D (residual loss) or -g / D for a given g (error loss);
 // dz3 = (dy wo) ⊙ [h3 > 0]; block partials of
 // (Σ dy x, Σ dy, Σ dy h3) for alpha, bo, wo.
@@ -1589,32 +2167,44 @@ struct dec_nn_s {
   DBuf<float2> ix;                                 // inference: (x, P x)
   DBuf<unsigned short> ih1, ih2;                   // inference: layer-1 and layer-2 rows
   DBuf<unsigned char> h1, hm1, h2, hm2, h3, dz;  // activation storage (bf16 or f32)
+  DBuf<float2> dm;                                 // (dy, signs of h3) per row
   DBuf<int32_t> idx;
   size_t cap_rows = 0;
-  int cap_prec = -1;
+  int cap_mode = -1;
 };
 
 namespace {
 
-void ensure(dec_nn_s &nn, size_t rows, int precise) {
-  if (rows <= nn.cap_rows && precise == nn.cap_prec) return;
-  size_t as = precise ? 4 : 2;
-  nn.x.alloc(rows);
-  nn.px.alloc(rows);
-  nn.y.alloc(rows);
-  nn.c.alloc(rows);
-  nn.drho.alloc(rows);
-  nn.eps.alloc(rows);
-  nn.tmp.alloc(rows);
-  nn.crs.alloc(rows);
-  nn.dg.alloc(rows * 2 * H);
-  for (auto *b : {&nn.h1, &nn.hm1, &nn.h2, &nn.hm2, &nn.h3, &nn.dz}) b->alloc(rows * H * as);
-  size_t parts = (rows + 255) / 256 + 64;
-  nn.part.alloc(parts * 2 * H * H);
-  nn.dpart.alloc(parts + 64);
+// How a batch runs: the tile kernels (BF16, P's rows of 1 to 8 slots), or one
+// kernel per operation with activations in BF16 (wider rows) or FP32.
+enum Mode { kTiles, kGeneral, kPrecise };
 
+template <class AT>
+Mode mode_of(const dec::NnLevel &L) {
+  if (sizeof(AT) == 4) return kPrecise;
+  auto narrow = [](const dec::NnLevel::Op &o) { return o.width >= 1 && o.width <= 8; };
+  return narrow(L.p) && narrow(L.pt) ? kTiles : kGeneral;
+}
+
+void ensure(dec_nn_s &nn, size_t rows, Mode mode) {
+  if (rows <= nn.cap_rows && mode == nn.cap_mode) return;
+  size_t as = mode == kPrecise ? 4 : 2;
+  for (auto *b : {&nn.x, &nn.px, &nn.y, &nn.drho, &nn.eps, &nn.crs}) b->alloc(rows);
+  size_t parts = (rows + 255) / 256 + 64;
+  nn.dpart.alloc(parts + 64);
+  for (auto *b : {&nn.h1, &nn.h2, &nn.h3, &nn.dz}) b->alloc(rows * H * as);
+  if (mode == kTiles) {
+    nn.dm.alloc(rows);
+    nn.part.alloc(static_cast<size_t>(kBackBlocks) * NP);
+  } else {
+    nn.c.alloc(rows);
+    nn.tmp.alloc(rows);
+    nn.dg.alloc(rows * 2 * H);
+    for (auto *b : {&nn.hm1, &nn.hm2}) b->alloc(rows * H * as);
+    nn.part.alloc(parts * 2 * H * H);
+  }
   nn.cap_rows = rows;
-  nn.cap_prec = precise;
+  nn.cap_mode = mode;
 }
 
 // out[j] = scale · Σ_p part[p·stride + off + j], j < width (kernels above)
@@ -1661,15 +2251,85 @@ void scale(dec_nn_s &nn, int n, int B, const float *r, hipStream_t st) {
   hipLaunchKernelGGL(k_scale_final, dim3(dec::nblocks(B, 64)), dim3(64), 0, st, n, B, nn.spart.p, nn.s.p);
 }
 
+int tile_count(int n, int B) {
+  long long t = static_cast<long long>((n + 63) / 64) * B;
+  if (t > 0x7fffffff / 64) fail(DEC_ERR_ARG, "learned smoother: batch too large");
+  return static_cast<int>(t);
+}
+
+// The forward pass on the tile kernels after the scales: h3 and y (or, with
+// the errors e, eps in place of y) and c, each where given.
+void forward_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, const float *e, unsigned short *h3,
+                   float *y, float *c_out, hipStream_t st) {
+  int n = L.n, tiles = tile_count(n, B);
+  auto *h1 = reinterpret_cast<unsigned short *>(nn.h1.p), *h2 = reinterpret_cast<unsigned short *>(nn.h2.p);
+  dim3 tg((tiles + 7) / 8 * 8), ig(dec::xcd_grid(tiles, kInfWaves));
+  DEC_ELL_WIDTH_SWITCH(L.p.width, if constexpr (W > 0) {
+    hipLaunchKernelGGL((k_fwd_input<W>), ig, dim3(TB), 0, st, n, B, L.p.col.p, L.p.val.p, r, nn.s.p, nn.th.p, nn.x.p,
+                       nn.px.p, h1);
+    hipLaunchKernelGGL((k_inf_layer2w<W>), tg, dim3(64), 0, st, n, B, L.p.col.p, L.p.val.p, h1, nn.th.p, h2);
+    hipLaunchKernelGGL((k_fwd_layer3w<W>), tg, dim3(64), 0, st, n, B, L.p.col.p, L.p.val.p, h2, nn.x.p, nn.th.p,
+                       nn.s.p, L.D.p, L.dmean, e, h3, y, c_out);
+  });
+}
+
+// Loss and gradient of a batch on the tile kernels.
+void loss_grad_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, const float *e, double *loss_out,
+                     hipStream_t st) {
+  int n = L.n;
+  ensure(nn, static_cast<size_t>(n) * B, kTiles);
+  scale(nn, n, B, r, st);
+  Acts<unsigned short> A = acts<unsigned short>(nn);
+  const float *th = nn.th.p;
+  forward_tiles(nn, L, B, r, e, A.h3, e ? nn.eps.p : nn.y.p, nullptr, st);
+  dim3 gv(dec::nblocks(n, TB), B);
+  int tiles = tile_count(n, B);
+  int blocks = std::min(kBackBlocks, dec::xcd_grid(tiles, kInfWaves));
+  if (!e) {
+    hipLaunchKernelGGL(k_loss, gv, dim3(TB), 0, st, n, B, L.a.width, L.a.col.p, L.a.val.p, nn.x.p, nn.y.p, L.D.p,
+                       nullptr, nn.drho.p, nn.dpart.p);
+    hipLaunchKernelGGL(k_head_back<false>, dim3(blocks), dim3(TB), 0, st, n, B, 0, L.at.width, L.at.col.p, L.at.val.p,
+                       nn.drho.p, nullptr, 1.0f, L.D.p, nn.x.p, A.h3, nn.dm.p, nn.part.p);
+  } else {
+    dim3 gc(dec::nblocks(L.nc, TB), B);
+    hipLaunchKernelGGL(k_bspmv, gc, dim3(TB), 0, st, L.nc, n, L.r.width, L.r.col.p, L.r.val.p, nn.eps.p, nn.crs.p);
+    hipLaunchKernelGGL(k_prolong_hp, gv, dim3(TB), 0, st, n, L.nc, L.pr.width, L.pr.col.p, L.pr.val.p, nn.crs.p,
+                       nn.eps.p, nn.dpart.p);
+    hipLaunchKernelGGL(k_bspmv, gc, dim3(TB), 0, st, L.nc, n, L.prt.width, L.prt.col.p, L.prt.val.p, nn.eps.p,
+                       nn.crs.p);
+    hipLaunchKernelGGL(k_head_back<true>, dim3(blocks), dim3(TB), 0, st, n, B, L.nc, L.rt.width, L.rt.col.p,
+                       L.rt.val.p, nn.eps.p, nn.crs.p, 2.0f * L.dmean / (static_cast<float>(n) * B), L.D.p, nn.x.p,
+                       A.h3, nn.dm.p, nn.part.p);
+  }
+  DEC_ELL_WIDTH_SWITCH(L.pt.width, if constexpr (W > 0) {
+    hipLaunchKernelGGL((k_layer_back<W, true>), dim3(blocks), dim3(TB), 0, st, n, B, L.pt.col.p, L.pt.val.p,
+                       static_cast<const unsigned short *>(nullptr), nn.dm.p, th + OWO, A.h2, th + OW3, A.dz,
+                       static_cast<const float *>(nullptr), static_cast<const float *>(nullptr), nn.part.p, OW3, OB2,
+                       OB3);
+    hipLaunchKernelGGL((k_layer_back<W, false>), dim3(blocks), dim3(TB), 0, st, n, B, L.pt.col.p, L.pt.val.p, A.dz,
+                       static_cast<const float2 *>(nullptr), static_cast<const float *>(nullptr), A.h1, th + OW2,
+                       static_cast<unsigned short *>(nullptr), nn.x.p, nn.px.p, nn.part.p, OW2, OB1, 0);
+  });
+  hipLaunchKernelGGL(k_reduce_params, dim3((NP + 63) / 64 + 1), dim3(1024), 0, st, blocks, nn.part.p, nn.grad.p,
+                     static_cast<int>(gv.x) * B, nn.dpart.p, 1.0 / (static_cast<double>(n) * B), loss_out);
+}
+
 template <class AT>
 void forward_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, float *c_out, float *u_add,
                hipStream_t st) {
   int n = L.n;
   size_t rows = static_cast<size_t>(n) * B;
-  ensure(nn, rows, sizeof(AT) == 4);
+  Mode mode = mode_of<AT>(L);
+  ensure(nn, rows, mode);
   Acts<AT> A = acts<AT>(nn);
   const float *th = nn.th.p;
   scale(nn, n, B, r, st);
+  if constexpr (sizeof(AT) == 2) {
+    if (mode == kTiles) {
+      forward_tiles(nn, L, B, r, nullptr, nullptr, nullptr, c_out, st);
+      return;
+    }
+  }
   dim3 gv(dec::nblocks(n, TB), B), gf(dec::nblocks(static_cast<long long>(n) * H, TB), B);
   hipLaunchKernelGGL(k_input<AT>, gv, dim3(TB), 0, st, n, L.p.width, L.p.col.p, L.p.val.p, r, nn.s.p, th, nn.x.p,
                      nn.px.p, A.h1);
@@ -1687,6 +2347,11 @@ template <class AT>
 // e: the B errors paired with the residuals (error loss), or NULL (residual loss).
 void loss_grad_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, const float *e, double *loss_out,
                  hipStream_t st) {
+  if (e && L.nc == 0) fail(DEC_ERR_ARG, "learned smoother: the error loss needs a coarser level below this one");
+  if (mode_of<AT>(L) == kTiles) {
+    loss_grad_tiles(nn, L, B, r, e, loss_out, st);
+    return;
+  }
   forward_t<AT>(nn, L, B, r, nullptr, nullptr, st);
   int n = L.n;
   int R = n * B;
@@ -1699,7 +2364,6 @@ void loss_grad_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, con
     hipLaunchKernelGGL(k_loss, gv, dim3(TB), 0, st, n, B, L.a.width, L.a.col.p, L.a.val.p, nn.x.p, nn.y.p, L.D.p,
                        nullptr, nn.drho.p, nn.dpart.p);
   } else {
-    if (L.nc == 0) fail(DEC_ERR_ARG, "learned smoother: the error loss needs a coarser level below this one");
     dim3 gc(dec::nblocks(L.nc, TB), B);
     hipLaunchKernelGGL(k_err, gv, dim3(TB), 0, st, n, L.dmean, e, nn.s.p, nn.y.p, L.D.p, nn.eps.p);
     hipLaunchKernelGGL(k_bspmv, gc, dim3(TB), 0, st, L.nc, n, L.r.width, L.r.col.p, L.r.val.p, nn.eps.p, nn.crs.p);
@@ -1804,7 +2468,7 @@ void nn_smooth(dec_nn_s &nn, int lvl, const float *r, float *u, hipStream_t s, b
         hipLaunchKernelGGL((k_inf_input_h<W>), dim3(dec::xcd_grid(n, TB)), dim3(TB), 0, s, n, NL.lidx.p,
                            NL.pi.val.p, NL.hoff.p, vorder ? NL.hrow_v.p : NL.hrow.p, rperm, r, nn.spart.p, nn.s.p,
                            x, nn.th.p, nn.ih1.p);
-        hipLaunchKernelGGL((k_inf_layer2w<W>), tg, dim3(64), 0, s, n, NL.pi.col.p, NL.pi.val.p, nn.ih1.p, nn.th.p,
+        hipLaunchKernelGGL((k_inf_layer2w<W>), tg, dim3(64), 0, s, n, 1, NL.pi.col.p, NL.pi.val.p, nn.ih1.p, nn.th.p,
                            nn.ih2.p);
         hipLaunchKernelGGL((k_inf_layer3w<W, float>), tg, dim3(64), 0, s, n, NL.pi.col.p, NL.pi.val.p, nn.ih2.p, x,
                            nn.th.p, nn.s.p, NL.Di.p, rperm, u);
@@ -1814,7 +2478,7 @@ void nn_smooth(dec_nn_s &nn, int lvl, const float *r, float *u, hipStream_t s, b
     DEC_ELL_WIDTH_SWITCH(NL.pi.width, if constexpr (W > 0) {
       hipLaunchKernelGGL((k_inf_input_c<W>), dim3(dec::xcd_grid(n, TB)), dim3(TB), 0, s, n, NL.pi.col.p,
                          NL.pi.val.p, rcol, rperm, r, nn.spart.p, nn.s.p, nn.ix.p, nn.th.p, nn.ih1.p);
-      hipLaunchKernelGGL((k_inf_layer2w<W>), tg, dim3(64), 0, s, n, NL.pi.col.p, NL.pi.val.p, nn.ih1.p, nn.th.p,
+      hipLaunchKernelGGL((k_inf_layer2w<W>), tg, dim3(64), 0, s, n, 1, NL.pi.col.p, NL.pi.val.p, nn.ih1.p, nn.th.p,
                          nn.ih2.p);
       hipLaunchKernelGGL((k_inf_layer3w<W, float2>), tg, dim3(64), 0, s, n, NL.pi.col.p, NL.pi.val.p, nn.ih2.p, nn.ix.p,
                          nn.th.p, nn.s.p, NL.Di.p, rperm, u);
