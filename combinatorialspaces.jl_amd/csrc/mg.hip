@@ -528,26 +528,22 @@ __global__ void k_sum_partials(const double *__restrict__ part, double *__restri
   if (threadIdx.x == 0) *out = s;
 }
 
-// Krylov.jl cg recurrence with device-resident scalars (warm start,
-// atol = rtol = sqrt(eps), zero-curvature exit).  γ and ‖p‖² are kept in two
-// slots: iteration `it` reads slot it & 1 and writes the other, so that the
-// blocks of one launch never see a value written in that launch.
+// Krylov.jl cg recurrence (warm start, atol = rtol = sqrt(eps), zero-curvature
+// exit), the multigrid's default smoother.  One reduction per step: with
+// p·Ap, Ap·Ap, r·Ap and r·r known, α = r·r / p·Ap and the next r·r is
+// r·r - 2 α r·Ap + α² Ap·Ap, from which β follows, so a step needs no second
+// reduction for β (the recurrence's own r·r enters α one step later).  Against
+// the usual two reductions the iterates agree to rounding.
+//
+// State of a smoothing on a level of several workgroups.  `stop` is the launch
+// (step + 1) whose scalars ended it (0: none); rbuf: which residual buffer
+// holds the last residual, xok: whether a step was added to x.  ‖p‖² is kept in
+// two slots: step `it` reads one and writes the other.
 struct CgState {
-  double gamma[2], pnorm2[2], rnorm, eps_stop, alpha, beta;
-  int done, iter;
+  double pnorm2[2], eps_stop;
+  int stop, rbuf, xok;
 };
 
-// Levels above kCgSmallRows rows: two launches per iteration.  The scalar
-// steps run inside the vector kernels: every block reduces all partial sums of
-// the previous launch itself, in one fixed order, so all blocks hold the same
-// γ, β and α, and block 0 alone writes the scalars back.  p is double-
-// buffered: the direction launch of iteration it > 0 forms p = r + β p_old for
-// its own rows into the other buffer, and its product evaluates r + β p_old at
-// every column, the expression the column's own row stores, so A p is the
-// product of the stored p without a launch in between.  The last step launch
-// adds the correction to u.  Against the four-launch sequence (product, dot,
-// α step, β step) the per-row values are the same expressions; only the dot
-// products add in another partition, so the iterates agree to rounding.
 constexpr int kCgBlocksMax = 1024;  // partial sums per reduction
 
 inline int cg_blocks(int n) { return std::min(kCgBlocksMax, dec::nblocks(n, kBlock)); }
@@ -576,88 +572,174 @@ __device__ double sum_partials(const double *__restrict__ part, int np) {
   return s;
 }
 
-// (A p)_i with p = r + β q evaluated at each column, summed in slot order.
-template <int W>
-__device__ __forceinline__ double row_dir(int n, int width, int i, const int *__restrict__ col,
-                                          const double *__restrict__ val, const double *__restrict__ r,
-                                          const double *__restrict__ q, double beta) {
-  double acc = 0.0;
-  if constexpr (W > 0) {
-    int c[W];
-    double v[W], rv[W], qv[W];
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-      size_t o = static_cast<size_t>(k) * n + i;
-      c[k] = col[o];
-      v[k] = val[o];
-    }
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-      int cc = c[k] < 0 ? 0 : c[k];
-      rv[k] = r[cc];
-      qv[k] = q[cc];
-    }
-#pragma unroll
-    for (int k = 0; k < W; k++)
-      if (c[k] >= 0) acc = acc + v[k] * (rv[k] + beta * qv[k]);
-  } else {
-    for (int k = 0; k < width; k++) {
-      size_t o = static_cast<size_t>(k) * n + i;
-      int cc = col[o];
-      if (cc < 0) break;
-      acc = acc + val[o] * (r[cc] + beta * q[cc]);
-    }
-  }
-  return acc;
+// Sum over the wavefront, the same value in every lane, by DPP row shifts and
+// broadcasts (no LDS round trips).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  long long b = __double_as_longlong(v);
+  int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, ROWS, 0xf, true);
+  int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, ROWS, 0xf, true);
+  return v + __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  long long b = __double_as_longlong(v);
+  int lo = __builtin_amdgcn_readlane(static_cast<int>(b), 63);
+  int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), 63);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
 }
 
-// *f as read by thread 0, the same for every thread of the block.  Block 0's
-// thread 0 may write *f later in the same launch; a block that reads that
-// value takes the exit its own scalars would take, and reading once keeps the
-// waves of a block on one path through its barriers.
-__device__ int block_flag(const int *f) {
-  __shared__ int v;
-  if (threadIdx.x == 0) v = *f;
+// The workgroup's sums of K values in every thread: the wavefronts' sums, then
+// those in order.  Successive calls (of any K ≤ KMAX) alternate between the
+// halves of red: a thread writes a half again only two calls later, after the
+// barrier of the call between, so one barrier per call suffices.
+template <int K, int WAVES, int KMAX>
+__device__ __forceinline__ void group_sums(double (&v)[K], double (*red)[WAVES * KMAX], int &half) {
+  static_assert(K <= KMAX, "a half holds WAVES * KMAX sums");
+#pragma unroll
+  for (int k = 0; k < K; k++) v[k] = wave_sum(v[k]);
+  double *h = red[half];
+  half ^= 1;
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < K; k++) h[(threadIdx.x >> 6) * K + k] = v[k];
+  }
   __syncthreads();
-  return v;
-}
-
-// r = b - A u, p = r, x = 0, and the partial sums of r·r.
-template <int W>
-__global__ void __launch_bounds__(kBlock)
-    k_cg2_start(int n, int width, const int *__restrict__ vcol, const double *__restrict__ vval,
-                const double *__restrict__ b, const double *__restrict__ u, double *__restrict__ r,
-                double *__restrict__ p, double *__restrict__ x, double *__restrict__ part) {
-  double acc = 0.0;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-    double ri = b[i] - dec_ell::row<W, double, double>(n, width, i, vcol, vval, u);
-    r[i] = ri;
-    p[i] = ri;
-    x[i] = 0.0;
-    acc = acc + ri * ri;
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    double t = h[k];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) t = t + h[w * K + k];
+    v[k] = t;
   }
-  double sum = block_sum<double>(acc);
-  if (threadIdx.x == 0) part[blockIdx.x] = sum;
 }
 
-// Iteration it's direction: at it = 0, γ = r·r, ‖r‖, the stopping threshold
-// and the immediate exit; at it > 0, ‖r‖ and the solved exit, β = γ_new / γ,
-// ‖p‖² and γ to slot it & 1, and p = r + β p_old.  Then A p and the partial
-// sums of p·Ap.
-template <int W>
+// ---- levels of several workgroups: one launch per step ---------------------
+// k_cg_start (r = b - A u and r·r), k_cg_step per step, k_cg_finish (the last
+// α, u += x, and before a coarse correction its right-hand side R r).  Every
+// workgroup adds the previous launch's partial sums itself, in one fixed order,
+// so all hold the same scalars; workgroup 0 alone writes the state.  A step
+// forms r and p of its own rows from the previous step's r, Ap and p, and the
+// same values at every column of its rows, the expressions the column's own row
+// stores, so A p needs no launch in between; r, p and Ap are double-buffered.
+// Levels of up to some 100,000 rows are bound by the launch and its chain of
+// dependent loads (4 to 6 µs each), not by bytes: a smoothing of three steps
+// with its restriction is 5 launches, where a direction and a step launch per
+// step, the residual and the restriction were 8 or 9.  dec_Δ⁻¹ on levels 3->7
+// (with the one-workgroup kernels below): 3.80 against 6.78 ms; five V-cycles
+// on 12,513 rows: 0.46 against 0.92 ms; as close to 64 bits as before (1e-12).
+constexpr int kCgWaves = kBlock / 64;
+
+// sums[k] = Σ part[k * kCgBlocksMax + j], j < nb
+template <int K>
+__device__ __forceinline__ void partial_sums(const double *__restrict__ part, int nb, double (&sums)[K],
+                                             double (*red)[kCgWaves * 4], int &half) {
+  double v[K];
+  const int t = static_cast<int>(threadIdx.x);
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    double q = part[k * kCgBlocksMax + min(t, nb - 1)];
+    v[k] = t < nb ? q : 0.0;
+  }
+  if (nb > kBlock) {  // all further loads at once
+    constexpr int kRun = kCgBlocksMax / kBlock - 1;
+    double q[K][kRun];
+#pragma unroll
+    for (int m = 0; m < kRun; m++)
+#pragma unroll
+      for (int k = 0; k < K; k++) q[k][m] = part[k * kCgBlocksMax + min(t + (m + 1) * kBlock, nb - 1)];
+#pragma unroll
+    for (int m = 0; m < kRun; m++)
+#pragma unroll
+      for (int k = 0; k < K; k++) v[k] = t + (m + 1) * kBlock < nb ? v[k] + q[k][m] : v[k];
+  }
+  group_sums<K, kCgWaves, 4>(v, red, half);
+#pragma unroll
+  for (int k = 0; k < K; k++) sums[k] = v[k];
+}
+
+template <int K>
+__device__ __forceinline__ void put_partials(double (&v)[K], int slot0, double *__restrict__ part,
+                                             double (*red)[kCgWaves * 4], int &half) {
+  group_sums<K, kCgWaves, 4>(v, red, half);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < K; k++) part[(slot0 + k) * kCgBlocksMax + blockIdx.x] = v[k];
+  }
+}
+
+// r = b - A u, with zc given (P an ELL of width 2) for u2 = u + P zc, which is
+// stored; the partial sums of r·r (slot 3); clears the state's stop.
+template <int W, bool FOLD>
 __global__ void __launch_bounds__(kBlock)
-    k_cg2_dir(CgState *st, int it, int n, int width, const int *__restrict__ vcol, const double *__restrict__ vval,
-              const double *__restrict__ r, const double *__restrict__ pold, double *__restrict__ p,
-              double *__restrict__ Ap, const double *__restrict__ part_rr, int nb, double *__restrict__ part_pap) {
-  if (it > 0 && block_flag(&st->done)) return;
+    k_cg_start(CgState *st, int n, int width, const int *__restrict__ vcol, const double *__restrict__ vval,
+               const double *__restrict__ b, const double *__restrict__ u, const int *__restrict__ pcol,
+               const double *__restrict__ pval, const double *__restrict__ zc, double *__restrict__ u2,
+               double *__restrict__ r, double *__restrict__ part) {
+  __shared__ double red[2][kCgWaves * 4];
+  int half = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->stop = 0;
+  double rr[1] = {0.0};
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    double s;
+    if constexpr (FOLD && W > 0) {
+      int c[W];
+      double v[W], uv[W];
+#pragma unroll
+      for (int k = 0; k < W; k++) {
+        size_t o = static_cast<size_t>(k) * n + i;
+        c[k] = vcol[o];
+        v[k] = vval[o];
+      }
+#pragma unroll
+      for (int k = 0; k < W; k++) uv[k] = prolonged(n, c[k] < 0 ? i : c[k], u, pcol, pval, zc);
+      u2[i] = prolonged(n, i, u, pcol, pval, zc);
+      s = 0.0;
+#pragma unroll
+      for (int k = 0; k < W; k++)
+        if (c[k] >= 0) s = s + v[k] * uv[k];
+    } else {
+      s = dec_ell::row<W, double, double>(n, width, i, vcol, vval, u);
+    }
+    double ri = b[i] - s;
+    r[i] = ri;
+    rr[0] = rr[0] + ri * ri;
+  }
+  put_partials<1>(rr, 3, part, red, half);
+}
+
+// r_i - α Ap_i
+__device__ __forceinline__ double next_r(double r, double a, double q) { return r - a * q; }
+
+// Step `it`.  IT0 (it = 0): p = r; Ap and the partial sums.  Else: the
+// scalars of step it - 1 from its partial sums (part_in), r = r_old - α Ap_old,
+// x += α p_old, p = r + β p_old (FIRST, it = 1: p_old = r_old and x = 0), then
+// Ap and the partial sums p·Ap, Ap·Ap, r·Ap, r·r.
+template <int W, bool IT0, bool FIRST>
+__global__ void __launch_bounds__(kBlock)
+    k_cg_step(CgState *st, int it, int n, int width, const int *__restrict__ vcol, const double *__restrict__ vval,
+              const double *__restrict__ r0, const double *__restrict__ p0, const double *__restrict__ q0,
+              double *__restrict__ r, double *__restrict__ p, double *__restrict__ q, double *__restrict__ x,
+              const double *__restrict__ part_in, int nb, double *__restrict__ part) {
+  __shared__ double red[2][kCgWaves * 4];
+  int half = 0;
+  const double eps = 2.220446049250313e-16;
   const int stride = gridDim.x * kBlock, i0 = blockIdx.x * kBlock + threadIdx.x;
-  // The thread's first row is loaded before the scalar step, which does not
-  // need it, so its loads are in flight while the partial sums are reduced.
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  int stop = 0;
+  if constexpr (!IT0) stop = st->stop;
+  // The thread's first row is loaded before the scalars, which it does not
+  // need, so its loads are in flight while the partial sums are added.
   constexpr int WP = W > 0 ? W : 1;
   int c0[WP];
-  double v0[WP], rc0[WP], qc0[WP], ri0 = 0.0, qi0 = 0.0;
+  double v0[WP], rc[WP], qc[WP], pc[WP];
+  const int ia = min(i0, n - 1);
   if constexpr (W > 0) {
-    int ia = min(i0, n - 1);
 #pragma unroll
     for (int k = 0; k < W; k++) {
       size_t o = static_cast<size_t>(k) * n + ia;
@@ -667,261 +749,375 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
     for (int k = 0; k < W; k++) {
       int cc = c0[k] < 0 ? 0 : c0[k];
-      rc0[k] = r[cc];
-      qc0[k] = pold[cc];
+      rc[k] = r0[cc];
+      if constexpr (!IT0) qc[k] = q0[cc];
+      if constexpr (!IT0 && !FIRST) pc[k] = p0[cc];
     }
-    ri0 = r[ia];
-    qi0 = pold[ia];
   }
-  double g = sum_partials(part_rr, nb);
-  double rn = sqrt(g);
-  bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-  double beta = 0.0;
-  if (it == 0) {
+  double ri0 = r0[ia], qi0 = 0.0, pi0 = 0.0, xi0 = 0.0;
+  if constexpr (!IT0) qi0 = q0[ia];
+  if constexpr (!IT0 && !FIRST) {
+    pi0 = p0[ia];
+    xi0 = x[ia];
+  }
+  double a = 0.0, beta = 0.0;
+  if constexpr (IT0) {
+    double g[1];
+    partial_sums<1>(part_in + 3 * kCgBlocksMax, nb, g, red, half);
     const double sq = 1.4901161193847656e-08;
-    double es = sq + sq * rn;
-    bool stop = (g == 0.0) || (rn <= es);
+    double rn = sqrt(g[0]), es = sq + sq * rn;
+    bool done = g[0] == 0.0 || rn <= es;
     if (lead) {
-      st->gamma[0] = g;
-      st->rnorm = rn;
       st->eps_stop = es;
-      st->pnorm2[0] = g;
-      st->iter = 0;
-      st->done = stop;
+      st->pnorm2[0] = g[0];
+      if (done) {
+        st->rbuf = 0;
+        st->xok = 0;
+        st->stop = 1;
+      }
     }
-    if (stop) return;
+    if (done) return;
   } else {
-    int c = (it - 1) & 1;
-    if (rn <= st->eps_stop || rn + 1.0 <= 1.0) {
+    // block 0 may set `stop` to it + 1 in this launch: only an earlier one ends it
+    if (stop != 0 && stop <= it) return;
+    double t[4];
+    partial_sums<4>(part_in, nb, t, red, half);
+    double pn2 = st->pnorm2[(it - 1) & 1], es = st->eps_stop;
+    if (t[0] <= eps * pn2 && fabs(t[0]) <= eps * pn2) {  // zero curvature: x and r stay
       if (lead) {
-        st->rnorm = rn;
-        st->iter += 1;
-        st->done = 2;  // solved: p is left as is
+        st->rbuf = (it - 1) & 1;
+        st->xok = it > 1;
+        st->stop = it + 1;
       }
       return;
     }
-    beta = g / st->gamma[c];
-    if (lead) {
-      st->rnorm = rn;
-      st->iter += 1;
-      st->beta = beta;
-      st->pnorm2[c ^ 1] = g + beta * beta * st->pnorm2[c];
-      st->gamma[c ^ 1] = g;
+    a = t[3] / t[0];
+    double gn = t[3] - 2.0 * a * t[2] + a * a * t[1];
+    gn = gn > 0.0 ? gn : 0.0;
+    double rn = sqrt(gn);
+    if (rn <= es || rn + 1.0 <= 1.0) {  // solved: the step still counts
+      for (int i = i0; i < n; i += stride) {
+        x[i] = (FIRST ? 0.0 : x[i]) + a * (FIRST ? r0[i] : p0[i]);
+        r[i] = next_r(r0[i], a, q0[i]);
+      }
+      if (lead) {
+        st->rbuf = it & 1;
+        st->xok = 1;
+        st->stop = it + 1;
+      }
+      return;
     }
+    beta = gn / t[3];
+    if (lead) st->pnorm2[it & 1] = gn + beta * beta * pn2;
   }
-  double acc = 0.0;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  auto own = [&](int i, double ro, double qo, double po, double xo, double s) {
+    double ri = IT0 ? ro : next_r(ro, a, qo), po_ = FIRST ? ro : po;
+    double pi = IT0 ? ri : ri + beta * po_;
+    if constexpr (!IT0) {
+      r[i] = ri;
+      p[i] = pi;
+      x[i] = xo + a * po_;
+    }
+    q[i] = s;
+    acc[0] = acc[0] + pi * s;
+    acc[1] = acc[1] + s * s;
+    acc[2] = acc[2] + ri * s;
+    acc[3] = acc[3] + ri * ri;
+  };
+  auto at = [&](double ro, double qo, double po) {
+    if constexpr (IT0) return ro;
+    double ri = next_r(ro, a, qo);
+    return ri + beta * (FIRST ? ro : po);
+  };
   int i = i0;
   if constexpr (W > 0) {
-    // the first row from the registers, with the sums of dec_ell::row and
-    // row_dir (slot order, the same products)
     if (i0 < n) {
-      double pi, api = 0.0;
-      if (it == 0) {
-        pi = qi0;
+      double s = 0.0;
 #pragma unroll
-        for (int k = 0; k < W; k++)
-          if (c0[k] >= 0) api = api + v0[k] * qc0[k];
-      } else {
-        pi = ri0 + beta * qi0;
-        p[i0] = pi;
-#pragma unroll
-        for (int k = 0; k < W; k++)
-          if (c0[k] >= 0) api = api + v0[k] * (rc0[k] + beta * qc0[k]);
-      }
-      Ap[i0] = api;
-      acc = acc + pi * api;
+      for (int k = 0; k < W; k++)
+        if (c0[k] >= 0) s = s + v0[k] * at(rc[k], IT0 ? 0.0 : qc[k], IT0 || FIRST ? 0.0 : pc[k]);
+      own(i0, ri0, qi0, pi0, xi0, s);
     }
     i += stride;
   }
   for (; i < n; i += stride) {
-    double pi, api;
-    if (it == 0) {
-      pi = pold[i];
-      api = dec_ell::row<W, double, double>(n, width, i, vcol, vval, pold);
+    double s = 0.0;
+    if constexpr (W > 0) {
+      int c[W];
+      double v[W], rv[W], qv[W], pv[W];
+#pragma unroll
+      for (int k = 0; k < W; k++) {
+        size_t o = static_cast<size_t>(k) * n + i;
+        c[k] = vcol[o];
+        v[k] = vval[o];
+      }
+#pragma unroll
+      for (int k = 0; k < W; k++) {
+        int cc = c[k] < 0 ? 0 : c[k];
+        rv[k] = r0[cc];
+        qv[k] = IT0 ? 0.0 : q0[cc];
+        pv[k] = IT0 || FIRST ? 0.0 : p0[cc];
+      }
+#pragma unroll
+      for (int k = 0; k < W; k++)
+        if (c[k] >= 0) s = s + v[k] * at(rv[k], qv[k], pv[k]);
     } else {
-      pi = r[i] + beta * pold[i];
-      p[i] = pi;
-      api = row_dir<W>(n, width, i, vcol, vval, r, pold, beta);
+      for (int k = 0; k < width; k++) {
+        size_t o = static_cast<size_t>(k) * n + i;
+        int cc = vcol[o];
+        if (cc < 0) break;
+        s = s + vval[o] * at(r0[cc], IT0 ? 0.0 : q0[cc], IT0 || FIRST ? 0.0 : p0[cc]);
+      }
     }
-    Ap[i] = api;
-    acc = acc + pi * api;
+    own(i, r0[i], IT0 ? 0.0 : q0[i], IT0 || FIRST ? 0.0 : p0[i], IT0 || FIRST ? 0.0 : x[i], s);
   }
-  double sum = block_sum<double>(acc);
-  if (threadIdx.x == 0) part_pap[blockIdx.x] = sum;
+  put_partials<4>(acc, 0, part, red, half);
 }
 
-// Iteration it's step: α = γ / p·Ap (zero-curvature exit), x += α p,
-// r -= α Ap and the partial sums of r·r; on the last iteration (LAST) u += x
-// instead (x as it stands when an exit came earlier).  The thread's first
-// element is loaded before the scalar step, so those loads are in flight
-// while the partial sums are reduced.
-template <bool LAST>
+// After the last step (steps of them): its α, u = u2 + x + α p, and with bc
+// given bc = R (r - α Ap) and a zero coarse iterate uc.  After an early exit u =
+// u2 + x and the residual is the one the exit left (ra / rb: the two buffers).
+template <int RW>
 __global__ void __launch_bounds__(kBlock)
-    k_cg2_step(CgState *st, int it, int n, double *__restrict__ x, const double *__restrict__ p,
-               double *__restrict__ r, const double *__restrict__ Ap, const double *__restrict__ part_pap, int nb,
-               double *__restrict__ part_rr, double *__restrict__ u) {
+    k_cg_finish(const CgState *__restrict__ st, int steps, int n, const double *u2,
+                const double *__restrict__ x, const double *__restrict__ p, const double *__restrict__ ra,
+                const double *__restrict__ rb, const double *__restrict__ q, const double *__restrict__ part, int nb,
+                double *u, int nc, int rwidth, const int *__restrict__ rcol,
+                const double *__restrict__ rval, double *__restrict__ bc, double *__restrict__ uc) {
+  __shared__ double red[2][kCgWaves * 4];
+  int half = 0;
   const double eps = 2.220446049250313e-16;
   const int stride = gridDim.x * kBlock, i0 = blockIdx.x * kBlock + threadIdx.x, ia = min(i0, n - 1);
-  double x0 = x[ia], p0 = p[ia], r0 = 0.0, a0 = 0.0, u0 = 0.0;
-  if constexpr (LAST) {
-    u0 = u[ia];
-  } else {
-    r0 = r[ia];
-    a0 = Ap[ia];
+  const int stop = st->stop, rbuf = st->rbuf, xok = st->xok;
+  const double pn2 = st->pnorm2[(steps - 1) & 1];
+  double u0 = u2[ia], x0 = steps > 1 ? x[ia] : 0.0, p0 = p[ia];
+  const double *r = ((steps - 1) & 1) ? rb : ra;
+  // the thread's first coarse row, in flight while the partial sums are added
+  constexpr int RP = RW > 0 ? RW : 1;
+  int c0[RP];
+  double v0[RP], rv0[RP], qv0[RP];
+  if constexpr (RW > 0) {
+    int ca = min(i0, nc - 1);
+#pragma unroll
+    for (int k = 0; k < RW; k++) {
+      size_t o = static_cast<size_t>(k) * nc + ca;
+      c0[k] = rcol[o];
+      v0[k] = rval[o];
+    }
+#pragma unroll
+    for (int k = 0; k < RW; k++) {
+      int cc = c0[k] < 0 ? 0 : c0[k];
+      rv0[k] = r[cc];
+      qv0[k] = q[cc];
+    }
   }
-  bool stop = block_flag(&st->done) != 0;
+  double t[4];
+  partial_sums<4>(part, nb, t, red, half);
   double a = 0.0;
-  if (!stop) {
-    double pAp = sum_partials(part_pap, nb);
-    int c = it & 1;
-    double pn2 = st->pnorm2[c];
-    if (pAp <= eps * pn2 && fabs(pAp) <= eps * pn2) {
-      if (blockIdx.x == 0 && threadIdx.x == 0) st->done = 1;
-      stop = true;
+  bool with_x = steps > 1;
+  if (stop != 0) {
+    with_x = xok != 0;
+    r = rbuf ? rb : ra;
+  } else if (!(t[0] <= eps * pn2 && fabs(t[0]) <= eps * pn2)) {
+    a = t[3] / t[0];
+  }
+  // (a = 0 adds nothing: p and Ap then hold values of an earlier smoothing,
+  // finite ones, or this one's)
+  auto step = [&](double ui, double xi, double pi) {
+    double xs = with_x ? xi : 0.0;
+    return (a != 0.0 ? xs + a * pi : xs) + ui;
+  };
+  if (i0 < n) u[i0] = step(u0, x0, p0);
+  for (int i = i0 + stride; i < n; i += stride) u[i] = step(u2[i], steps > 1 ? x[i] : 0.0, p[i]);
+  if (!bc) return;
+  int i = i0;
+  if constexpr (RW > 0) {
+    if (stop == 0) {
+      if (i0 < nc) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < RW; k++)
+          if (c0[k] >= 0) s = s + v0[k] * (a != 0.0 ? next_r(rv0[k], a, qv0[k]) : rv0[k]);
+        bc[i0] = s;
+        uc[i0] = 0.0;
+      }
+      i += stride;
+    }
+  }
+  for (; i < nc; i += stride) {
+    double s = 0.0;
+    if constexpr (RW > 0) {
+      int c[RW];
+      double v[RW], rv[RW], qv[RW];
+#pragma unroll
+      for (int k = 0; k < RW; k++) {
+        size_t o = static_cast<size_t>(k) * nc + i;
+        c[k] = rcol[o];
+        v[k] = rval[o];
+      }
+#pragma unroll
+      for (int k = 0; k < RW; k++) {
+        int cc = c[k] < 0 ? 0 : c[k];
+        rv[k] = r[cc];
+        qv[k] = q[cc];
+      }
+#pragma unroll
+      for (int k = 0; k < RW; k++)
+        if (c[k] >= 0) s = s + v[k] * (a != 0.0 ? next_r(rv[k], a, qv[k]) : rv[k]);
     } else {
-      a = st->gamma[c] / pAp;
-      if (blockIdx.x == 0 && threadIdx.x == 0) st->alpha = a;
+      for (int k = 0; k < rwidth; k++) {
+        size_t o = static_cast<size_t>(k) * nc + i;
+        int cc = rcol[o];
+        if (cc < 0) break;
+        s = s + rval[o] * (a != 0.0 ? next_r(r[cc], a, q[cc]) : r[cc]);
+      }
     }
+    bc[i] = s;
+    uc[i] = 0.0;
   }
-  if constexpr (LAST) {
-    if (i0 < n) {
-      double xi = stop ? x0 : x0 + a * p0;
-      u[i0] = xi + u0;
-    }
-    for (int i = i0 + stride; i < n; i += stride) {
-      double xi = stop ? x[i] : x[i] + a * p[i];
-      u[i] = xi + u[i];
-    }
-    return;
-  }
-  if (stop) return;
-  double acc = 0.0;
-  if (i0 < n) {
-    x[i0] = x0 + a * p0;
-    double ri = r0 - a * a0;
-    r[i0] = ri;
-    acc = acc + ri * ri;
-  }
-  for (int i = i0 + stride; i < n; i += stride) {
-    x[i] = x[i] + a * p[i];
-    double ri = r[i] - a * Ap[i];
-    r[i] = ri;
-    acc = acc + ri * ri;
-  }
-  double sum = block_sum<double>(acc);
-  if (threadIdx.x == 0) part_rr[blockIdx.x] = sum;
 }
 
-// The CG smoother (the recurrence of k_cg2_*) on a level of at most
-// kCgSmallRows rows, as one workgroup of kCgThreads threads: thread t owns
-// rows t + kCgThreads k (k < R) and holds their slots, values, x, r and A p
-// in registers for the whole smoothing; p lives in LDS, so after the first
-// residual every product is LDS gathers only.  Each dot product is one
-// workgroup reduction in a fixed order (waves, then the waves' sums).  One
-// launch per smoothing in place of 1 + 2 steps launches.  Its dot products
-// add in another order than the multi-launch partition, so its iterates
-// agree with those of the multi-launch smoother to rounding.
-constexpr int kCgThreads = 1024;
-constexpr int kCgRowsPerThread = 3;  // slots and values of 3 rows of up to 7 fit in 128 VGPRs
-constexpr int kCgSmallRows = kCgThreads * kCgRowsPerThread;
+// ---- small levels: one workgroup, in registers and LDS ---------------------
+// A level of at most kCgSmallRows rows of at most kCgWidth slots: thread t of
+// kCgThreads owns rows t + kCgThreads k (k < R) and holds their columns (16
+// bits each) and values in registers; p lives in LDS, so a product is LDS
+// gathers only.  512 threads of up to 256 registers hold 7 rows each, where 1024
+// threads of 128 held 3 (with 32-bit columns).  A smoothing of three steps takes
+// 7.0 µs at 642 rows, 12.9 at 2,562 and 14.6 at 3,185 (1.2 to 2.3 µs a step: the
+// product's LDS gathers, one reduction, two barriers), against 11 and 15.1 µs at
+// 642 and 2,562 rows with two reductions by LDS shuffles per step; a level of
+// 10,242 rows on several workgroups takes 20.
+constexpr int kCgThreads = 512;
+constexpr int kCgWidth = 7;
+constexpr int kCgRowsMax = 7;
+constexpr int kCgSmallRows = kCgThreads * kCgRowsMax;
+constexpr int kCgCoarseRows = 2;  // rows per thread of the coarsest level in the tail
+constexpr int kCgGroupWaves = kCgThreads / 64;
 
-// The workgroup's sum of v: each wave's shuffle tree, then the 16 wave sums
-// in order, read by every thread.  Successive calls alternate between the two
-// halves of red[2][16]: a thread writes a half again only two calls later,
-// after the barrier of the call between, by which time every thread has read
-// it, so one barrier per call suffices.
-__device__ double wg_sum(double v, double (*red)[kCgThreads / 64], int &half) {
-  for (int off = 32; off > 0; off >>= 1) v = v + __shfl_down(v, off, 64);
-  double *h = red[half];
-  half ^= 1;
-  if ((threadIdx.x & 63) == 0) h[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double t = 0.0;
-  for (int k = 0; k < kCgThreads / 64; k++) t = t + h[k];
-  return t;
+struct CgLevel {
+  int n, width;
+  const int *col;
+  const double *val;
+};
+
+// *(p + off bytes): a uniform base and a 32-bit offset per lane
+template <class T>
+__device__ __forceinline__ T at_byte(const T *__restrict__ p, unsigned int off) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + off);
 }
 
-// Σ_s v[s] x[c[s]] over the slots with c[s] ≥ 0, in slot order (the sum of
-// dec_ell::row).
-template <int W>
-__device__ __forceinline__ double row_regs(const int (&c)[W], const double (&v)[W], const double *x) {
-  double xv[W];
+template <int R>
+struct CgRows {
+  unsigned int c[R][4];  // columns' byte offsets (8 c) in pairs; a pad is the row itself with value 0
+  double v[R][kCgWidth];
+};
+
+template <int R>
+__device__ __forceinline__ void load_cg_rows(CgRows<R> &o, const CgLevel &L) {
 #pragma unroll
-  for (int s = 0; s < W; s++) xv[s] = x[c[s] < 0 ? 0 : c[s]];
+  for (int k = 0; k < R; k++) {
+    int i = static_cast<int>(threadIdx.x) + k * kCgThreads, ia = min(i, L.n - 1);
+    unsigned int c[kCgWidth + 1];
+    c[kCgWidth] = 0;
+#pragma unroll
+    for (int s = 0; s < kCgWidth; s++) {
+      unsigned int q = static_cast<unsigned int>(min(s, L.width - 1) * L.n + ia);
+      int cc = at_byte(L.col, 4u * q);
+      double vv = at_byte(L.val, 8u * q);
+      bool has = s < L.width && cc >= 0 && i < L.n;
+      c[s] = 8u * static_cast<unsigned int>(has ? cc : ia);
+      o.v[k][s] = has ? vv : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++) o.c[k][s] = c[2 * s] | (c[2 * s + 1] << 16);
+  }
+}
+
+// v, as a value the compiler knows nothing about: what is computed from it
+// inside a loop is not kept in registers across the loop
+__device__ __forceinline__ unsigned int opaque(unsigned int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// Σ_s v[s] x[c[s]] in slot order, by fused multiply-adds
+template <int R>
+__device__ __forceinline__ double cg_row(const CgRows<R> &o, int k, const double *x) {
+  double xv[kCgWidth];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    unsigned int c = opaque(o.c[k][j]);
+    xv[2 * j] = at_byte(x, c & 0xffffu);
+    if (2 * j + 1 < kCgWidth) xv[2 * j + 1] = at_byte(x, c >> 16);
+  }
   double acc = 0.0;
 #pragma unroll
-  for (int s = 0; s < W; s++)
-    if (c[s] >= 0) acc = acc + v[s] * xv[s];
+  for (int s = 0; s < kCgWidth; s++) acc = __builtin_fma(o.v[k][s], xv[s], acc);
   return acc;
 }
 
-template <int W, int R>
-__global__ void __launch_bounds__(kCgThreads)
-    k_cg_smooth_small(int n, const int *__restrict__ vcol, const double *__restrict__ vval,
-                      const double *__restrict__ b, double *__restrict__ u, int steps) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  double *p = reinterpret_cast<double *>(smem_raw);
-  __shared__ double red[2][kCgThreads / 64];
-  int half = 0;
-  int c[R][W];
-  double v[R][W], x[R], r[R], Ap[R];
-#pragma unroll
-  for (int k = 0; k < R; k++) {
-    int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
-#pragma unroll
-    for (int s = 0; s < W; s++) {
-      size_t o = static_cast<size_t>(s) * n + (i < n ? i : 0);
-      c[k][s] = i < n ? vcol[o] : -1;
-      v[k][s] = vval[o];
-    }
-  }
-  double acc = 0.0;
-#pragma unroll
-  for (int k = 0; k < R; k++) {
-    int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
-    x[k] = 0.0;
-    r[k] = 0.0;
-    Ap[k] = 0.0;
-    if (i < n) {
-      r[k] = b[i] - row_regs<W>(c[k], v[k], u);
-      p[i] = r[k];
-      acc = acc + r[k] * r[k];
-    }
-  }
-  double gamma = wg_sum(acc, red, half);
-  double rnorm = sqrt(gamma);
+typedef double CgRed[2][kCgGroupWaves * 3];
+
+// Up to `steps` CG steps from the residual r (each thread's rows), added to
+// u; r is the residual after them.  p: n values of LDS, free on entry (a barrier
+// has passed since their last use).
+template <int R>
+__device__ __forceinline__ void cg_run(const CgRows<R> &o, int n, int steps, double (&u)[R], double (&r)[R], double *p,
+                                       CgRed &red, int &half) {
   const double sq = 1.4901161193847656e-08, eps = 2.220446049250313e-16;
-  const double eps_stop = sq + sq * rnorm;
-  double pnorm2 = gamma;
-  bool done = (gamma == 0.0) || (rnorm <= eps_stop);
-  for (int it = 0; it < steps && !done; it++) {
-    __syncthreads();  // p complete
-    double pap = 0.0;
+  double g[1] = {0.0};
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+    if (i < n) p[i] = r[k];
+    g[0] = g[0] + r[k] * r[k];
+  }
+  group_sums<1, kCgGroupWaves, 3>(g, red, half);
+  double gamma = g[0], pnorm2 = gamma;
+  const double rn = sqrt(gamma), es = sq + sq * rn;
+  if (gamma == 0.0 || rn <= es) return;
+  // ‖r‖ ≤ es or ‖r‖ + 1 ≤ 1, as tests of r·r: no square root in the steps
+  const double solved = fmax(es * es, 1.23e-32);
+  // (the sums' barrier has made p complete)
+  for (int it = 0; it < steps; it++) {
+    const double over = 1.0 / gamma;  // ready before β needs it
+    double q[R], t[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+      int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+      q[k] = 0.0;
+      if (i < n) {
+        q[k] = cg_row<R>(o, k, p);
+        t[0] = t[0] + p[i] * q[k];
+        t[1] = t[1] + q[k] * q[k];
+        t[2] = t[2] + r[k] * q[k];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // rows one after the other: registers
+    }
+    group_sums<3, kCgGroupWaves, 3>(t, red, half);
+    if (t[0] <= eps * pnorm2 && fabs(t[0]) <= eps * pnorm2) return;
+    double a = gamma / t[0];
+    double gn = gamma - 2.0 * a * t[2] + a * a * t[1];
 #pragma unroll
     for (int k = 0; k < R; k++) {
       int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
       if (i < n) {
-        Ap[k] = row_regs<W>(c[k], v[k], p);
-        pap = pap + p[i] * Ap[k];
+        u[k] = u[k] + a * p[i];
+        r[k] = r[k] - a * q[k];
       }
     }
-    double pAp = wg_sum(pap, red, half);
-    if (pAp <= eps * pnorm2 && fabs(pAp) <= eps * pnorm2) break;
-    double a = gamma / pAp;
-    double rr = 0.0;
+    if (it + 1 == steps) return;
+    if (!(gn > 1e-6 * gamma)) {
+      // too much cancelled: the sum itself (the same branch in every thread)
+      g[0] = 0.0;
 #pragma unroll
-    for (int k = 0; k < R; k++) {
-      int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
-      if (i < n) {
-        x[k] = x[k] + a * p[i];
-        r[k] = r[k] - a * Ap[k];
-        rr = rr + r[k] * r[k];
-      }
+      for (int k = 0; k < R; k++) g[0] = g[0] + r[k] * r[k];
+      group_sums<1, kCgGroupWaves, 3>(g, red, half);
+      gn = g[0];
     }
-    double gn = wg_sum(rr, red, half);
-    double rn = sqrt(gn);
-    if (rn <= eps_stop || rn + 1.0 <= 1.0) break;
-    double beta = gn / gamma;
+    if (gn <= solved) return;
+    double beta = gn * over;
     pnorm2 = gn + beta * beta * pnorm2;
     gamma = gn;
 #pragma unroll
@@ -929,11 +1125,162 @@ __global__ void __launch_bounds__(kCgThreads)
       int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
       if (i < n) p[i] = r[k] + beta * p[i];
     }
+    __syncthreads();
+  }
+}
+
+// r = b - A u of the thread's rows, u in LDS (complete)
+template <int R>
+__device__ __forceinline__ void cg_residual(const CgRows<R> &o, int n, const double *__restrict__ b, const double *u,
+                                            double (&r)[R]) {
+  double bv[R];
+  const int t = static_cast<int>(opaque(threadIdx.x));
+#pragma unroll
+  for (int k = 0; k < R; k++) bv[k] = at_byte(b, 8u * static_cast<unsigned int>(min(t + k * kCgThreads, n - 1)));
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+    r[k] = i < n ? bv[k] - cg_row<R>(o, k, u) : 0.0;
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// The transfer to the next coarser level: R's rows (nc) and P's.
+struct CgTransfer {
+  int nc, rwidth, pwidth;
+  const int *rcol, *pcol;
+  const double *rval, *pval;
+};
+
+// u += P z of the thread's rows, z in LDS or memory
+template <int R>
+__device__ __forceinline__ void cg_prolong(const CgTransfer &T, int n, const double *z, double (&u)[R]) {
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    int ia = min(static_cast<int>(opaque(threadIdx.x)) + k * kCgThreads, n - 1);
+    u[k] = u[k] + (T.pwidth == 2 ? dec_ell::row<2, double, double>(n, T.pwidth, ia, T.pcol, T.pval, z)
+                                 : dec_ell::row<0, double, double>(n, T.pwidth, ia, T.pcol, T.pval, z));
+  }
+}
+
+// row i of R r, r in LDS
+__device__ __forceinline__ double cg_restrict(const CgTransfer &T, int i, const double *r) {
+  return T.rwidth == 7 ? dec_ell::row<7, double, double>(T.nc, T.rwidth, i, T.rcol, T.rval, r)
+                       : dec_ell::row<0, double, double>(T.nc, T.rwidth, i, T.rcol, T.rval, r);
+}
+
+// `reps` smoothings of one small level, one after the other: u += x.  With zc
+// given they start from u + P zc; with bc given the residual is restricted
+// (bc = R r, and a zero coarse iterate uc).
+template <int R>
+__global__ void __launch_bounds__(kCgThreads)
+    k_cg_small(CgLevel L, const double *__restrict__ b, double *__restrict__ u, int steps, int reps, CgTransfer T,
+               const double *__restrict__ zc, double *__restrict__ bc, double *__restrict__ uc) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double *p = reinterpret_cast<double *>(smem_raw);
+  __shared__ CgRed red;
+  int half = 0;
+  CgRows<R> o;
+  load_cg_rows<R>(o, L);
+  double uv[R], r[R];
+#pragma unroll
+  for (int k = 0; k < R; k++) uv[k] = u[min(static_cast<int>(threadIdx.x) + k * kCgThreads, L.n - 1)];
+  if (zc) cg_prolong<R>(T, L.n, zc, uv);
+  for (int q = 0; q < reps; q++) {
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+      int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+      if (i < L.n) p[i] = uv[k];
+    }
+    __syncthreads();
+    cg_residual<R>(o, L.n, b, p, r);
+    __syncthreads();
+    cg_run<R>(o, L.n, steps, uv, r, p, red, half);
+    __syncthreads();
   }
 #pragma unroll
   for (int k = 0; k < R; k++) {
     int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
-    if (i < n) u[i] = x[k] + u[i];
+    if (i < L.n) {
+      u[i] = uv[k];
+      if (bc) p[i] = r[k];
+    }
+  }
+  if (!bc) return;
+  __syncthreads();
+  for (int i = threadIdx.x; i < T.nc; i += kCgThreads) {
+    bc[i] = cg_restrict(T, i, p);
+    uc[i] = 0.0;
+  }
+}
+
+// `cycles` μ-cycles of the two coarsest levels A and C (C of at most 1024 rows)
+// in one launch: each smooths A, restricts, smooths C once or twice (twice, the
+// W-cycle's, in the first `wcycles` of them), prolongs and smooths A again.
+// Both levels' rows stay in registers throughout; vectors pass through LDS.  In
+// place of six or seven launches a cycle that each loaded a level again: 44 µs
+// for a W-cycle's two visits of 2,562 and 642 rows, against about 110.
+template <int R, int RC>
+__global__ void __launch_bounds__(kCgThreads)
+    k_cg_tail(CgLevel A, CgLevel C, const double *__restrict__ b, double *__restrict__ u, int steps, int cycles,
+              int wcycles, CgTransfer T) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double *pa = reinterpret_cast<double *>(smem_raw), *pc = pa + A.n;
+  __shared__ CgRed red;
+  int half = 0;
+  CgRows<R> oa;
+  CgRows<RC> oc;
+  load_cg_rows<R>(oa, A);
+  double ua[R];
+#pragma unroll
+  for (int k = 0; k < R; k++) ua[k] = u[min(static_cast<int>(threadIdx.x) + k * kCgThreads, A.n - 1)];
+  load_cg_rows<RC>(oc, C);
+  for (int cyc = 0; cyc < cycles; cyc++) {
+    double r[R], rc[RC], uc[RC];
+    auto smooth_a = [&]() {
+#pragma unroll
+      for (int k = 0; k < R; k++) {
+        int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+        if (i < A.n) pa[i] = ua[k];
+      }
+      __syncthreads();
+      cg_residual<R>(oa, A.n, b, pa, r);
+      __syncthreads();
+      cg_run<R>(oa, A.n, steps, ua, r, pa, red, half);
+      __syncthreads();
+    };
+    smooth_a();
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+      int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+      if (i < A.n) pa[i] = r[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RC; k++) {
+      int i = static_cast<int>(opaque(threadIdx.x)) + k * kCgThreads;
+      rc[k] = cg_restrict(T, min(i, C.n - 1), pa);
+      if (i >= C.n) rc[k] = 0.0;
+      uc[k] = 0.0;
+    }
+    // C starts at zero: its residual is b_c, then what the steps leave
+    for (int v = 0; v < (cyc < wcycles ? 2 : 1); v++) {
+      cg_run<RC>(oc, C.n, steps, uc, rc, pc, red, half);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < RC; k++) {
+      int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+      if (i < C.n) pc[i] = uc[k];
+    }
+    __syncthreads();
+    cg_prolong<R>(T, A.n, pc, ua);
+    smooth_a();
+  }
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    int i = static_cast<int>(threadIdx.x) + k * kCgThreads;
+    if (i < A.n) u[i] = ua[k];
   }
 }
 
@@ -1359,7 +1706,7 @@ struct dec_mg_s {
   double omega = 2.0 / 3.0;
   DBuf<double> part, part2, scal;  // reduction partials, scalar outputs
   DBuf<CgState> cg;
-  DBuf<double> cgx, cgp, cgp2, cgAp;  // CG vectors (finest size; p double-buffered)
+  DBuf<double> cgx, cgr, cgp, cgp2, cgAp, cgAp2;  // CG vectors (finest size; r, p and Ap double-buffered)
   int fuse_from = -1;           // first level handled by the fused coarse kernel
   DBuf<LevelDesc<double>> desc64;
   DBuf<LevelDesc<float>> desc32;
@@ -1847,8 +2194,8 @@ void finish_hierarchy(dec_mg_s &mg, const std::vector<dec::HostCsr> &As, std::ve
     mg.hdesc64 = d64;
     mg.hdesc32 = d32;
   }
-  mg.part.alloc(kCgBlocksMax);  // also the dot partials (kDotBlocks of them)
-  mg.part2.alloc(kCgBlocksMax);
+  mg.part.alloc(4 * kCgBlocksMax);  // also the dot partials (kDotBlocks of them)
+  mg.part2.alloc(4 * kCgBlocksMax);
   mg.scal.alloc(8);
   mg.rpart.alloc(static_cast<size_t>(dec::nblocks(mg.lv[0]->n, kBlock)));
   if (hipHostMalloc(reinterpret_cast<void **>(&mg.hnorm), sizeof(double) * (kNormSlots + 1), hipHostMallocDefault) !=
@@ -1858,10 +2205,7 @@ void finish_hierarchy(dec_mg_s &mg, const std::vector<dec::HostCsr> &As, std::ve
     if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) fail(DEC_ERR_HIP, "hipEventCreate failed");
   mg.cg.alloc(1);
   int nf = mg.lv[0]->n;
-  mg.cgx.alloc(nf);
-  mg.cgp.alloc(nf);
-  mg.cgp2.alloc(nf);
-  mg.cgAp.alloc(nf);
+  for (auto *v : {&mg.cgx, &mg.cgr, &mg.cgp, &mg.cgp2, &mg.cgAp, &mg.cgAp2}) v->alloc(nf);
 }
 
 void env_switches(dec_mg_s &mg) {
@@ -2003,31 +2347,100 @@ void dot(dec_mg_s &mg, int n, const double *x, const double *y, double *out, con
   hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kBlock), 0, s, mg.part.p, out, done);
 }
 
-// cg(A, b, u; itmax = steps) as in Multigrid.jl:860 (float64 only), on a
-// level above kCgSmallRows rows: 1 + 2 steps launches (the residual with the
-// start, then a direction and a step launch per iteration).
-void cg_smooth(dec_mg_s &mg, Level &L, const double *b, double *u, int steps, hipStream_t s) {
-  if (steps <= 0) return;
+// cg(A, b, u; itmax = steps) as in Multigrid.jl:860 (float64 only) on a level of
+// several workgroups: 2 + steps launches.  zc: the coarse correction, u + P zc
+// the iterate it starts from (P's ELL of width 2); coarse: the next coarser
+// level, whose b and zero iterate the last launch writes (R of the residual).
+void cg_smooth(dec_mg_s &mg, Level &L, const double *b, double *u, int steps, const double *zc, Level *coarse,
+               hipStream_t s) {
   int n = L.n, nb = cg_blocks(n);
   CgState *st = mg.cg.p;
-  double *x = mg.cgx.p, *Ap = mg.cgAp.p, *r = L.d.t.p;
-  double *pb[2] = {mg.cgp.p, mg.cgp2.p};
-  DEC_ELL_WIDTH_SWITCH(L.width, hipLaunchKernelGGL((k_cg2_start<W>), dim3(nb), dim3(kBlock), 0, s, n, L.width,
-                                                   L.vcol.p, L.d.vval.p, b, u, r, pb[0], x, mg.part.p));
-  for (int it = 0; it < steps; it++) {
-    // iteration it's p is pb[it & 1]; the direction launch forms it from
-    // pb[(it - 1) & 1] (at it = 0, pb[0] already holds p = r and is only read)
-    double *pold = it == 0 ? pb[0] : pb[(it + 1) & 1], *pnew = it == 0 ? pb[1] : pb[it & 1];
-    DEC_ELL_WIDTH_SWITCH(L.width, hipLaunchKernelGGL((k_cg2_dir<W>), dim3(nb), dim3(kBlock), 0, s, st, it, n,
-                                                     L.width, L.vcol.p, L.d.vval.p, r, pold, pnew, Ap, mg.part.p,
-                                                     nb, mg.part2.p));
-    if (it + 1 == steps)
-      hipLaunchKernelGGL(k_cg2_step<true>, dim3(nb), dim3(kBlock), 0, s, st, it, n, x, pb[it & 1], r, Ap,
-                         mg.part2.p, nb, mg.part.p, u);
+  double *x = mg.cgx.p, *rb[2] = {L.d.t.p, mg.cgr.p}, *pb[2] = {mg.cgp.p, mg.cgp2.p}, *qb[2] = {mg.cgAp.p, mg.cgAp2.p};
+  double *part[2] = {mg.part.p, mg.part2.p};
+  double *u2 = zc ? L.d.r.p : u;
+  DEC_ELL_WIDTH_SWITCH(L.width, {
+    if (zc)
+      hipLaunchKernelGGL((k_cg_start<W, true>), dim3(nb), dim3(kBlock), 0, s, st, n, L.width, L.vcol.p, L.d.vval.p, b,
+                         u, L.pcol.p, L.d.pval.p, zc, u2, rb[0], part[1]);
     else
-      hipLaunchKernelGGL(k_cg2_step<false>, dim3(nb), dim3(kBlock), 0, s, st, it, n, x, pb[it & 1], r, Ap,
-                         mg.part2.p, nb, mg.part.p, u);
+      hipLaunchKernelGGL((k_cg_start<W, false>), dim3(nb), dim3(kBlock), 0, s, st, n, L.width, L.vcol.p, L.d.vval.p,
+                         b, u, static_cast<const int *>(nullptr), static_cast<const double *>(nullptr),
+                         static_cast<const double *>(nullptr), static_cast<double *>(nullptr), rb[0], part[1]);
+  });
+  for (int it = 0; it < steps; it++) {
+    int w = it & 1, o = w ^ 1;
+    const double *r0 = it == 0 ? rb[0] : rb[o], *p0 = it <= 1 ? rb[0] : pb[o];
+#define DEC_CG_STEP(A, B)                                                                                              \
+  DEC_ELL_WIDTH_SWITCH(L.width, hipLaunchKernelGGL((k_cg_step<W, A, B>), dim3(nb), dim3(kBlock), 0, s, st, it, n,  \
+                                                   L.width, L.vcol.p, L.d.vval.p, r0, p0, qb[o], rb[w], pb[w], qb[w], \
+                                                   x, part[o], nb, part[w]))
+    if (it == 0) {
+      DEC_CG_STEP(true, false);
+    } else if (it == 1) {
+      DEC_CG_STEP(false, true);
+    } else {
+      DEC_CG_STEP(false, false);
+    }
+#undef DEC_CG_STEP
   }
+  int w = (steps - 1) & 1;
+  const double *p = steps == 1 ? rb[0] : pb[w];
+  int nc = coarse ? L.nc : 0, rw = coarse ? L.rwidth : 0;
+  DEC_ELL_WIDTH_SWITCH(rw, hipLaunchKernelGGL((k_cg_finish<W>), dim3(nb), dim3(kBlock), 0, s, st, steps, n, u2, x, p,
+                                              rb[0], rb[1], qb[w], part[w], nb, u, nc, rw, L.rcol.p, L.d.rval.p,
+                                              coarse ? coarse->d.b.p : nullptr, coarse ? coarse->d.u.p : nullptr));
+}
+
+// Levels that one workgroup smooths (k_cg_small, k_cg_tail).
+inline bool cg_small(const Level &L) { return L.n <= kCgSmallRows && L.width >= 1 && L.width <= kCgWidth; }
+
+inline CgLevel cg_level(Level &L) { return CgLevel{L.n, L.width, L.vcol.p, L.d.vval.p}; }
+
+// LAUNCH with R = the least of 1, 2, 4, 6 and 7 rows per thread that hold n rows
+#define DEC_CG_ROWS_SWITCH(n, LAUNCH)                                   \
+  do {                                                                  \
+    if ((n) <= kCgThreads) { constexpr int R = 1; LAUNCH; }             \
+    else if ((n) <= 2 * kCgThreads) { constexpr int R = 2; LAUNCH; }    \
+    else if ((n) <= 4 * kCgThreads) { constexpr int R = 4; LAUNCH; }    \
+    else if ((n) <= 6 * kCgThreads) { constexpr int R = 6; LAUNCH; }    \
+    else { constexpr int R = kCgRowsMax; LAUNCH; }                      \
+  } while (0)
+
+inline CgTransfer cg_transfer(Level &L) {
+  return CgTransfer{L.nc, L.rwidth, L.pwidth, L.rcol.p, L.pcol.p, L.d.rval.p, L.d.pval.p};
+}
+
+// zc, coarse: as for cg_smooth (P's ELL of any width)
+void cg_small_smooth(Level &L, const double *b, double *u, int steps, int reps, const double *zc, Level *coarse,
+                     hipStream_t s) {
+  size_t lds = static_cast<size_t>(L.n) * sizeof(double);
+  DEC_CG_ROWS_SWITCH(L.n, hipLaunchKernelGGL((k_cg_small<R>), dim3(1), dim3(kCgThreads), lds, s, cg_level(L), b, u,
+                                             steps, reps, cg_transfer(L), zc, coarse ? coarse->d.b.p : nullptr,
+                                             coarse ? coarse->d.u.p : nullptr));
+}
+
+// Whether the cycles of level lvl run as k_cg_tail.
+bool cg_tail_at(const dec_mg_s &mg, int lvl) {
+  int nl = static_cast<int>(mg.lv.size());
+  if (!mg.use_fused || mg.alg != DEC_SMOOTH_CG || mg.steps == 0 || mg.coarse_direct || lvl != nl - 2) return false;
+  const Level &A = *mg.lv[lvl], &C = *mg.lv[nl - 1];
+  return cg_small(A) && cg_small(C) && C.n <= kCgCoarseRows * kCgThreads;
+}
+
+// `cycles` μ-cycles of level lvl, the first `wcycles` of them with two visits of
+// the coarsest level.
+void cg_tail(dec_mg_s &mg, int lvl, double *u, const double *b, int cycles, int wcycles, hipStream_t s) {
+  Level &A = *mg.lv[lvl], &C = *mg.lv[lvl + 1];
+  size_t lds = static_cast<size_t>(A.n + C.n) * sizeof(double);
+#define DEC_CG_TAIL(RC)                                                                                              \
+  DEC_CG_ROWS_SWITCH(A.n, hipLaunchKernelGGL((k_cg_tail<R, RC>), dim3(1), dim3(kCgThreads), lds, s, cg_level(A),    \
+                                             cg_level(C), b, u, mg.steps, cycles, wcycles, cg_transfer(A)))
+  if (C.n <= kCgThreads) {
+    DEC_CG_TAIL(1);
+  } else {
+    DEC_CG_TAIL(kCgCoarseRows);
+  }
+#undef DEC_CG_TAIL
 }
 
 inline bool learned_on(const dec_mg_s &mg) { return mg.nn && mg.learned && mg.learned_active; }
@@ -2045,6 +2458,9 @@ constexpr int kPrefetchMaxRows = 200000;
 // (measured: 6.8 against 9.0 µs at 40,962 rows, 18.5 against 10.6 µs at
 // 163,842, where evaluating shared fine rows twice costs more than a launch).
 constexpr int kFusedRestrictMaxRows = 50000;
+// The CG smoother's first launch after the coarse correction adds it itself on
+// levels up to this many rows.
+constexpr int kCgFoldMaxRows = 100000;
 
 // Rows per thread of the prefetching sweep for this level's blocks (1 or 2
 // with up to 256 threads), or 0 when it does not apply (wide rows, or a
@@ -2084,7 +2500,7 @@ void launch_block_gs_pf(Level &L, LevelVals<T> &V, int R, int nthr, size_t lds, 
 
 template <class T>
 void smooth(dec_mg_s &mg, int lvl, Level &L, const T *b, T *u, bool post, bool u_zero, hipStream_t s,
-            const T *zc = nullptr) {
+            const T *zc = nullptr, Level *coarse = nullptr) {
   int steps = mg.steps;
   if (steps == 0) return;
   LevelVals<T> &V = vals<T>(L);
@@ -2103,15 +2519,8 @@ void smooth(dec_mg_s &mg, int lvl, Level &L, const T *b, T *u, bool post, bool u
   }
   if (mg.alg == DEC_SMOOTH_CG) {
     if constexpr (sizeof(T) == 8) {
-      if (L.n <= kCgSmallRows && L.width >= 1 && L.width <= 7) {
-        size_t lds = static_cast<size_t>(L.n) * sizeof(double);  // p
-        DEC_ELL_WIDTH_SWITCH(L.width, if constexpr (W > 0) {
-          hipLaunchKernelGGL((k_cg_smooth_small<W, kCgRowsPerThread>), dim3(1), dim3(kCgThreads), lds, s, L.n,
-                             L.vcol.p, L.d.vval.p, b, u, steps);
-        });
-      } else {
-        cg_smooth(mg, L, b, u, steps, s);
-      }
+      if (cg_small(L)) cg_small_smooth(L, b, u, steps, 1, zc, coarse, s);
+      else cg_smooth(mg, L, b, u, steps, zc, coarse, s);
     } else {
       fail(DEC_ERR_UNSUPPORTED, "the CG smoother runs in float64 only");
     }
@@ -2259,12 +2668,21 @@ void mu_cycle(dec_mg_s &mg, int lvl, T *u, const T *b, int mu, bool u_zero, hipS
     coarse_solve<T>(mg, L, b, u, s);
     return;
   }
-  smooth<T>(mg, lvl, L, b, u, false, u_zero, s);
+  // the CG smoother restricts its residual itself
+  bool cg_on = sizeof(T) == 8 && mg.alg == DEC_SMOOTH_CG && mg.steps > 0;
+  if constexpr (sizeof(T) == 8)
+    if (cg_tail_at(mg, lvl)) {
+      cg_tail(mg, lvl, u, b, 1, mu > 1 ? 1 : 0, s);
+      return;
+    }
+  smooth<T>(mg, lvl, L, b, u, false, u_zero, s, nullptr, cg_on && lvl < nl - 1 ? mg.lv[lvl + 1].get() : nullptr);
   if (lvl >= nl - 1) return;
   Level &C = *mg.lv[lvl + 1];
   LevelVals<T> &V = vals<T>(L);
   LevelVals<T> &CV = vals<T>(C);
-  if (L.n <= kFusedRestrictMaxRows && L.rwidth <= 8) {
+  if (cg_on) {
+    // b and u of the coarser level are in place
+  } else if (L.n <= kFusedRestrictMaxRows && L.rwidth <= 8) {
     DEC_ELL_WIDTH_SWITCH(L.width, hipLaunchKernelGGL((k_residual_restrict<W, T>), G(8LL * L.nc), dim3(kBlock), 0, s,
                                                      L.nc, L.rwidth, L.rcol.p, V.rval.p, L.n, L.width, L.vcol.p,
                                                      V.vval.p, b, u, CV.b.p, CV.u.p));
@@ -2273,14 +2691,23 @@ void mu_cycle(dec_mg_s &mg, int lvl, T *u, const T *b, int mu, bool u_zero, hipS
     DEC_ELL_WIDTH_SWITCH(L.rwidth, hipLaunchKernelGGL((k_restrict<W, T>), G(L.nc), dim3(kBlock), 0, s, L.nc,
                                                       L.rwidth, L.rcol.p, V.rval.p, V.r.p, CV.b.p, CV.u.p));
   }
-  mu_cycle<T>(mg, lvl + 1, CV.u.p, CV.b.p, mu, true, s);
-  if (mu > 1) mu_cycle<T>(mg, lvl + 1, CV.u.p, CV.b.p, mu - 1, false, s);
+  bool tail = false;
+  if constexpr (sizeof(T) == 8) {
+    tail = cg_tail_at(mg, lvl + 1);
+    // (both visits of the two coarsest levels in one launch)
+    if (tail) cg_tail(mg, lvl + 1, CV.u.p, CV.b.p, mu > 1 ? 2 : 1, mu > 2 ? 2 : (mu > 1 ? 1 : 0), s);
+  }
+  if (!tail) {
+    mu_cycle<T>(mg, lvl + 1, CV.u.p, CV.b.p, mu, true, s);
+    if (mu > 1) mu_cycle<T>(mg, lvl + 1, CV.u.p, CV.b.p, mu - 1, false, s);
+  }
   // the hybrid smoother's first post-sweep applies the prolongation itself
   // (on the prefetching sweep only: there the extra loads join the load
   // phase; on the streaming sweep of the largest level they cost more than
   // the separate launch, measured 37 against 18 + 6.5 µs at 655,362 rows)
   bool fold = mg.alg == DEC_SMOOTH_BLOCK_GS && mg.steps > 0 && L.pwidth == 2 && prefetch_rows(L) > 0 &&
               L.n <= kPrefetchMaxRows && !(sizeof(T) == 4 && learned_on(mg) && learned_rows(mg, L.n));
+  fold = fold || (cg_on && (cg_small(L) || (L.pwidth == 2 && L.width >= 1 && L.width <= 8 && L.n <= kCgFoldMaxRows)));
   if (!fold)
     DEC_ELL_WIDTH_SWITCH(L.pwidth, hipLaunchKernelGGL((k_prolong_add<W, T>), G(L.n), dim3(kBlock), 0, s, L.n,
                                                       L.pwidth, L.pcol.p, V.pval.p, CV.u.p, u));
@@ -2301,8 +2728,14 @@ void fmg_rec(dec_mg_s &mg, int lvl, const double *b, double *z, int mu, int cycl
     DEC_ELL_WIDTH_SWITCH(L.pwidth, hipLaunchKernelGGL((k_prolong_add<W, double>), G(L.n), dim3(kBlock), 0, s, L.n,
                                                       L.pwidth, L.pcol.p, L.d.pval.p, C.d.u.p, z));
   }
-  if (lvl > 0)
+  if (lvl == 0) return;
+  if (cg_tail_at(mg, lvl)) {
+    if (cycles > 0) cg_tail(mg, lvl, z, b, cycles, mu > 1 ? cycles : 0, s);
+  } else if (lvl == nl - 1 && mg.alg == DEC_SMOOTH_CG && mg.steps > 0 && !mg.coarse_direct && cg_small(L)) {
+    if (cycles > 0) cg_small_smooth(L, b, z, mg.steps, cycles, nullptr, nullptr, s);
+  } else {
     for (int c = 0; c < cycles; c++) mu_cycle<double>(mg, lvl, z, b, mu, false, s);
+  }
 }
 
 // The caller's finest-level vectors in the hierarchy's numbering: b into
