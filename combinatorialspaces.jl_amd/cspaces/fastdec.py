@@ -37,10 +37,29 @@ class Barycenter:
     code = L.DEC_BARYCENTER
 
 
-def _torch():
-    import torch
+class _Torch:
+    """torch (imported on first use) and what a call on the hot path needs of it."""
 
-    return torch
+    module = None
+    Tensor = None
+
+    @classmethod
+    def load(cls):
+        import torch
+
+        cls.Tensor = torch.Tensor
+        try:
+            raw, dev = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+            # the handle of torch.cuda.current_stream(), without the Stream object around it
+            cls.current_stream = staticmethod(lambda: raw(dev()))
+        except AttributeError:
+            cls.current_stream = staticmethod(lambda: torch.cuda.current_stream().cuda_stream)
+        cls.module = torch
+        return torch
+
+
+def _torch():
+    return _Torch.module or _Torch.load()
 
 
 def _dtype_code(cast_float):
@@ -58,9 +77,11 @@ def _torch_dtype(code):
 
 
 def _stream(stream):
-    torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return c_void_p(s.cuda_stream)
+    """The handle of `stream` (None: torch's current one), as ctypes passes it to a void pointer."""
+    if stream is not None:
+        return stream.cuda_stream
+    _torch()
+    return _Torch.current_stream()
 
 
 def _hodge(h):
@@ -404,6 +425,7 @@ class Operator:
         r, c, c2 = c_int64(), c_int64(), c_int64()
         check(lib().dec_op_shape(h, ctypes.byref(r), ctypes.byref(c), ctypes.byref(c2)))
         self.rows, self.cols, self.cols2 = r.value, c.value, c2.value
+        self._hv, self._apply = h.value, lib().dec_op_apply
 
     @property
     def handle(self):
@@ -419,31 +441,39 @@ class Operator:
                 lib().dec_op_destroy(self._h)
             except Exception:
                 pass
-            self._h = None
+            self._h = self._hv = None
 
     def _check_form(self, x, n, name):
-        torch = _torch()
-        if not isinstance(x, torch.Tensor) or not x.is_cuda:
+        if (isinstance(x, _Torch.Tensor) and x.is_cuda and x.dtype == self.dtype and x.numel() == n
+                and x.is_contiguous()):
+            return
+        if not isinstance(x, _torch().Tensor) or not x.is_cuda:
             raise TypeError(f"{name} must be a GPU torch tensor")
         if x.dtype != self.dtype:
             raise TypeError(f"{name} has dtype {x.dtype}, operator computes in {self.dtype}")
-        if x.numel() != n or not x.is_contiguous():
-            raise ValueError(f"{name} must be contiguous with {n} entries, got {tuple(x.shape)}")
+        raise ValueError(f"{name} must be contiguous with {n} entries, got {tuple(x.shape)}")
 
+    # One application costs the host about 5 µs, half of it the kernel launch; on
+    # meshes of up to some 100,000 vertices that is what it takes.  So the checks
+    # are one expression, the output's allocation, the stream and the pointers go
+    # to the library without objects around them, and nothing is looked up twice.
     def apply(self, x, y=None, out=None, stream=None):
-        torch = _torch()
         self._check_form(x, self.cols, "x")
         if self.cols2:
             if y is None:
                 raise TypeError("this operator takes two forms")
             self._check_form(y, self.cols2, "y")
         if out is None:
-            out = torch.empty(self.rows, dtype=self.dtype, device=x.device)
+            if type(x) is _Torch.Tensor:
+                out = x.new_empty(self.rows)
+            else:
+                out = _torch().empty(self.rows, dtype=self.dtype, device=x.device)
         else:
             self._check_form(out, self.rows, "out")
-        check(lib().dec_op_apply(self._h, c_void_p(x.data_ptr()),
-                                 c_void_p(y.data_ptr()) if y is not None else None,
-                                 c_void_p(out.data_ptr()), _stream(stream)))
+        status = self._apply(self._hv, x.data_ptr(), None if y is None else y.data_ptr(), out.data_ptr(),
+                             _Torch.current_stream() if stream is None else stream.cuda_stream)
+        if status:
+            check(status)
         return out
 
     __call__ = apply
@@ -455,7 +485,7 @@ class Operator:
                 raise TypeError("this operator takes two forms")
             self._check_form(y, self.cols2, "y")
         self._check_form(out, self.rows, "out")
-        return self._h.value, x.data_ptr(), (y.data_ptr() if y is not None else None), out.data_ptr()
+        return self._hv, x.data_ptr(), (y.data_ptr() if y is not None else None), out.data_ptr()
 
     def __matmul__(self, x):
         return self.apply(x)
@@ -674,8 +704,6 @@ def apply_many(items, stream=None):
     items = list(items)
     if not items:
         return
-    args = [op._args(x, y, out) for op, x, y, out in items]
-    n = len(args)
-    arr = lambda vals: (c_void_p * n)(*vals)  # noqa: E731
-    check(lib().dec_op_apply_many(n, arr([a[0] for a in args]), arr([a[1] for a in args]),
-                                  arr([a[2] for a in args]), arr([a[3] for a in args]), _stream(stream)))
+    ops, xs, ys, outs = zip(*[op._args(x, y, out) for op, x, y, out in items])
+    arr = c_void_p * len(items)
+    check(lib().dec_op_apply_many(len(items), arr(*ops), arr(*xs), arr(*ys), arr(*outs), _stream(stream)))
