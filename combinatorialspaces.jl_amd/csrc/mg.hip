@@ -20,6 +20,7 @@
 
 using dec::DBuf;
 using dec::fail;
+using dec::wave_sum;
 
 namespace {
 
@@ -287,28 +288,6 @@ template <>
 struct Vec2T<float> {
   using type = float2;
 };
-
-// Sum over the wavefront, the same value in every lane, by DPP row shifts and
-// broadcasts (no LDS round trips).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-  long long b = __double_as_longlong(v);
-  int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, ROWS, 0xf, true);
-  int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, ROWS, 0xf, true);
-  return v + __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-__device__ __forceinline__ double wave_sum(double v) {
-  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
-  v = dpp_add<0x112, 0xf>(v);
-  v = dpp_add<0x114, 0xf>(v);
-  v = dpp_add<0x118, 0xf>(v);
-  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-  long long b = __double_as_longlong(v);
-  int lo = __builtin_amdgcn_readlane(static_cast<int>(b), 63);
-  int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), 63);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
 
 // The sweep from the level's panels: every load is issued before the colour
 // phases, which touch only registers and LDS.  A block's panel holds its rows

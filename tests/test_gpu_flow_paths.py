@@ -46,9 +46,9 @@ def test_lie_equals_its_parts(O, cs, name, dtype):
 @pytest.mark.parametrize("dtype", ["f64", "f32"])
 @pytest.mark.parametrize("name", MESHES)
 def test_dual_laplacian1_equals_its_parts(O, cs, name, dtype):
-    """Δᵈ(1) x = M x + N ⋆1⁻¹ x with its factors applied one by one.  The
-    products' rows hold at most 24 terms, so forming them differs from applying
-    the factors by a few dozen roundings of the largest entries."""
+    """Δᵈ(1) x = ⋆1 d0 (⋆0⁻¹ d̃1 x) + d̃0 ⋆2 d1 ⋆1⁻¹ x with its factors applied one by
+    one.  The products' rows hold few terms, so forming them differs from applying
+    the factors by a few roundings of the largest entries."""
     import torch
 
     td = torch.float64 if dtype == "f64" else torch.float32
@@ -57,7 +57,7 @@ def test_dual_laplacian1_equals_its_parts(O, cs, name, dtype):
     x = to_dev(torch, O.uniform_form(83, L1.rows), td)
     y = L1(x)
     z = x.clone()
-    L1.apply(z, out=z)                              # in place: the separate launches
+    L1.apply(z, out=z)                              # in place
     assert torch.equal(z, y)
     H = cs.GeometricHodge
     op = lambda k, f, *a: f(k, gm, *a, cast_float=torch.float64)  # noqa: E731
