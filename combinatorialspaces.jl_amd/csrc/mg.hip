@@ -455,39 +455,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Rows held in registers with a level's whole iterate in LDS (the coarse tail).
-template <int W, class T, int R>
-struct OwnedRows {
-  int v[R], c[R];
-  int col[R][W];
-  T val[R][W], halo[R][W], b[R];
-};
-
-// The colour phases of one sweep over the owned rows (x: the block's iterate in LDS).
-template <int W, class T, int R>
-__device__ __forceinline__ void sweep_owned(const OwnedRows<W, T, R> &o, T *x, int r0, int nr, int ncolors,
-                                            bool reverse) {
-  for (int ci = 0; ci < ncolors; ci++) {
-    int c = reverse ? ncolors - 1 - ci : ci;
-#pragma unroll
-    for (int i = 0; i < R; i++) {
-      if (o.c[i] != c) continue;
-      int v = o.v[i];
-      T s = static_cast<T>(0), d = static_cast<T>(0);
-#pragma unroll
-      for (int q = 0; q < W; q++) {
-        int cq = o.col[i][q];
-        if (cq < 0) continue;
-        unsigned loc = static_cast<unsigned>(cq - r0);
-        if (cq == v) d = o.val[i][q];
-        else s = s + o.val[i][q] * (loc < static_cast<unsigned>(nr) ? x[loc] : o.halo[i][q]);
-      }
-      x[v - r0] = (o.b[i] - s) / d;
-    }
-    __syncthreads();
-  }
-}
-
 // ---- set-up: what a level keeps besides its vertex-ordered ELL --------------
 
 // the rows of an ELL in another order: row p is row order[p]
@@ -585,18 +552,21 @@ __global__ void k_perm_scatter(int n, const int *__restrict__ perm, const T *__r
 
 // u += Z r with Z stored column-major (ZT[j * n + i] = Z[i, j]), in two
 // launches so that the whole chip streams Z: the columns are cut into chunks of
-// kCoarseChunk, one workgroup of 64 rows per (row tile, chunk) writes
+// coarse_chunk(n), one workgroup of 64 rows per (row tile, chunk) writes
 // part[c * n + i] = Σ_{j in chunk c, ascending} Z[i, j] r[j], and the second
 // pass adds Σ_c part[c * n + i] (c ascending) to u.  The fused coarse tail
 // uses the same two sums in the same order.
-constexpr int kCoarseChunk = 64;
+// (16 columns where the coarse tail, whose threads hold a chunk's part of a row in
+// registers, can be the one that multiplies: its LDS ends at 1,792 beside 3,072 rows.
+// 64 above, for fewer partial sums.)
+__host__ __device__ inline int coarse_chunk(int n) { return n <= 1792 ? 16 : 64; }
 
 template <class T>
 __global__ void __launch_bounds__(64)
     k_coarse_partial(int n, const T *__restrict__ ZT, const T *__restrict__ r, T *__restrict__ part) {
   int i = blockIdx.x * 64 + threadIdx.x;
-  int j0 = blockIdx.y * kCoarseChunk;
-  int j1 = min(n, j0 + kCoarseChunk);
+  int j0 = blockIdx.y * coarse_chunk(n);
+  int j1 = min(n, j0 + coarse_chunk(n));
   if (i >= n) return;
   T acc = static_cast<T>(0);
 #pragma unroll 16
@@ -607,6 +577,7 @@ __global__ void __launch_bounds__(64)
 template <class T>
 __device__ __forceinline__ T coarse_sum(int n, int nchunks, int i, const T *__restrict__ part) {
   T acc = static_cast<T>(0);
+#pragma unroll 8
   for (int c = 0; c < nchunks; c++) acc = acc + part[static_cast<size_t>(c) * n + i];
   return acc;
 }
@@ -617,7 +588,7 @@ __global__ void k_coarse_finish(int n, int nchunks, const T *__restrict__ part, 
   if (i < n) u[i] = u[i] + coarse_sum(n, nchunks, i, part);
 }
 
-inline int coarse_chunks(int n) { return (n + kCoarseChunk - 1) / kCoarseChunk; }
+__host__ __device__ inline int coarse_chunks(int n) { return (n + coarse_chunk(n) - 1) / coarse_chunk(n); }
 
 template <class T>
 __device__ double block_sum(double v) {
@@ -1630,7 +1601,7 @@ __global__ void __launch_bounds__(kFuseThreads)
   } else {
     const LevelDesc<T> &C = Ls[nl - 1];
     T *uc = nl - 1 == l0 ? u0 : C.u;
-    int nch = (C.n + kCoarseChunk - 1) / kCoarseChunk;
+    int nch = coarse_chunks(C.n);
     for (int i = threadIdx.x; i < C.n; i += blockDim.x) uc[i] = uc[i] + coarse_sum(C.n, nch, i, part);
     __syncthreads();
   }
@@ -1647,102 +1618,264 @@ __global__ void __launch_bounds__(kFuseThreads)
   }
 }
 
-// The coarse tail when it is one smoothed level A (at most 3 x 1024 rows,
-// ELL width 1-8) above the dense coarsest level C, in Gauss-Seidel V-cycles:
-// the same phases and per-row arithmetic as k_fused_vcycle with A's rows held
-// in registers (thread t owns positions t + 1024 i) and its vectors in LDS, so
-// the colour phases wait on no memory access.
-//   phase 1: A's pre-smoothing, residual and restriction; C's b and its
-//            residual (C's iterate starts at zero, so that residual is b).
-//   phase 2: C's correction from k_coarse_partial's chunks, the prolongation
-//            to A and A's post-smoothing.
-template <int W, class T, int R>
-__global__ void __launch_bounds__(kFuseThreads)
-    k_tail2(const LevelDesc<T> A, const LevelDesc<T> C, T *__restrict__ uA, const T *__restrict__ bA, int steps,
-            int phase, const T *__restrict__ part) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  int n = A.n;
-  T *x = reinterpret_cast<T *>(smem_raw);
-  T *w = x + n;  // phase 1: A's residual; phase 2: C's correction
-  OwnedRows<W, T, R> o;
-#pragma unroll
-  for (int i = 0; i < R; i++) {
-    int q = static_cast<int>(threadIdx.x) + i * kFuseThreads;
-    o.v[i] = -1;
-    o.c[i] = -1;
-    if (q >= n) continue;
-    int c = 0;
-    while (c + 1 < A.ncolors && q >= A.cstart[c + 1]) c++;
-    o.c[i] = c;
-    o.v[i] = A.rowid[q];
-#pragma unroll
-    for (int sl = 0; sl < W; sl++) {
-      size_t off = static_cast<size_t>(sl) * n + q;
-      o.col[i][sl] = A.col[off];
-      o.val[i][sl] = A.val[off];
+// The coarse tail in Gauss-Seidel V-cycles above a dense coarsest level: for each
+// smoothed level A of at most 3 x 1024 rows of 1-8 slots a launch on the way down
+// and one on the way up, with A's rows in registers (thread t owns positions
+// t + 1024 i of the rows sorted by colour) and its vectors in LDS, so that the
+// colour phases wait on no memory access.  A row is one uint4 (the 12-bit numbers
+// of its up to 7 off-diagonal slots; beside the first the diagonal's place among
+// them, in the last 16 bits the row's own number and colour), the off-diagonal values
+// slot by slot and the diagonal; nothing that is loaded names another load.
+//   k_tail_down: A's pre-smoothing, residual and restriction.  Above the dense
+//     coarsest level C also its direct solve Z r (C's iterate starts at zero):
+//     Z is too much for one workgroup, so one for every 16 of C's rows does the whole
+//     of A's part by itself and then its rows of Z r, and a launch is saved.
+//   k_tail_up: the prolongation of C's correction to A and A's post-smoothing.
+// Every sum is k_fused_vcycle's and k_coarse_partial's, bit for bit.
+// Bound by the colour phases (a barrier each) and one round trip for the loads.
+// Measured with 2,562 rows above 642, three sweeps either way, float64: 14.3 + 10.2
+// µs, where rows that were read by number, their colours searched in a table and
+// the product in a launch of its own took 16.8 + 4.7 + 16.8; 1,700 rows above
+// 437, two sweeps, float32: 9.3 + 5.7, against 11 + 4.7 + 11.
+template <class T>
+struct Tail {
+  int n, nc, ncolors, rwidth, pwidth;
+  const uint4 *idx;
+  const T *off, *diag;
+  const int *rcol, *pcol;
+  const T *rval, *pval;
+  const T *ZT;  // null: C is not the dense coarsest level
+};
+
+constexpr int kTailRows = 3 * kFuseThreads;  // 12-bit numbers, three rows a thread
+constexpr int kTailZ = 16;                   // rows of C in a workgroup
+
+// x (later the chunks' parts of 16 rows of Z r), w, and C's right-hand side
+__host__ __device__ inline int tail_x(int n, int nc) {
+  int parts = coarse_chunks(nc) * kTailZ;
+  return n > parts ? n : parts;
+}
+inline size_t tail_lds(int n, int nc, size_t bytes) {
+  return (static_cast<size_t>(tail_x(n, nc)) + n + nc) * bytes;
+}
+
+__global__ void k_build_tail(const LevelDesc<double> A, int S, uint4 *__restrict__ idx, double *__restrict__ off,
+                             double *__restrict__ diag) {
+  int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= A.n) return;
+  unsigned int v = static_cast<unsigned int>(A.rowid[q]), w[8], at = 0, k = 0, c = 0;
+  while (static_cast<int>(c) + 1 < A.ncolors && q >= A.cstart[c + 1]) c++;
+  for (int j = 0; j < 8; j++) w[j] = v;
+  for (int sl = 0; sl < A.width; sl++) {
+    size_t o = static_cast<size_t>(sl) * A.n + q;
+    int cc = A.col[o];
+    if (cc < 0) continue;
+    if (static_cast<unsigned int>(cc) == v) {
+      at = k;
+      diag[q] = A.val[o];
+    } else if (k < static_cast<unsigned int>(S)) {  // (the host has checked that no row has more)
+      w[k] = static_cast<unsigned int>(cc);
+      off[static_cast<size_t>(k) * A.n + q] = A.val[o];
+      k++;
     }
-    o.b[i] = bA[o.v[i]];
   }
-  if (phase == 1) {
-    // the restriction row this thread forms at the end, loaded up front
-    // (one coarse row per thread when R is at most 8 wide and C has at most
-    // 1024 rows; else the rows are read at the end)
-    bool rpre = A.rwidth <= 8 && A.nc <= kFuseThreads;
-    int rcl[8];
-    T rvl[8];
-    int ri = threadIdx.x;
-#pragma unroll
-    for (int sl = 0; sl < 8; sl++) {
-      rcl[sl] = -1;
-      rvl[sl] = static_cast<T>(0);
-      if (rpre && ri < A.nc && sl < A.rwidth) {
-        size_t off = static_cast<size_t>(sl) * A.nc + ri;
-        rcl[sl] = A.rcol[off];
-        rvl[sl] = A.rval[off];
-      }
-    }
-    for (int i = threadIdx.x; i < n; i += kFuseThreads) x[i] = uA[i];
-    __syncthreads();
-    for (int it = 0; it < steps; it++) sweep_owned<W, T, R>(o, x, 0, n, A.ncolors, false);
+  for (; k < static_cast<unsigned int>(S); k++) off[static_cast<size_t>(k) * A.n + q] = 0.0;
+  w[0] |= at << 12;
+  w[7] |= c << 12;
+  idx[q] = make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
+}
+
+template <int S, class T, int R>
+struct TailRows {
+  uint4 ix[R];
+  T off[R][S], d[R], b[R];
+
+  __device__ __forceinline__ void load(const Tail<T> &A) {
 #pragma unroll
     for (int i = 0; i < R; i++) {
-      if (o.v[i] < 0) continue;
-      T acc = static_cast<T>(0);
+      int q = static_cast<int>(threadIdx.x) + i * kFuseThreads, qc = min(q, A.n - 1);
+      ix[i] = A.idx[qc];
+      if (q >= A.n) ix[i].w = 0xf0000000u;  // no colour
+      d[i] = A.diag[qc];
 #pragma unroll
-      for (int sl = 0; sl < W; sl++)
-        if (o.col[i][sl] >= 0) acc = acc + o.val[i][sl] * x[o.col[i][sl]];
-      w[o.v[i]] = o.b[i] - acc;
+      for (int k = 0; k < S; k++) off[i][k] = A.off[static_cast<size_t>(k) * A.n + qc];
     }
-    __syncthreads();
-    if (rpre) {
-      if (ri < A.nc) {
-        T bc = static_cast<T>(0);
-#pragma unroll
-        for (int sl = 0; sl < 8; sl++)
-          if (rcl[sl] >= 0) bc = bc + rvl[sl] * w[rcl[sl]];
-        C.b[ri] = bc;
-        C.r[ri] = bc;
-      }
-    } else {
-      for (int i = threadIdx.x; i < A.nc; i += kFuseThreads) {
-        T bc = A.rwidth == 7 ? dec_ell::row<7, T, T>(A.nc, A.rwidth, i, A.rcol, A.rval, w)
-                             : dec_ell::row<0, T, T>(A.nc, A.rwidth, i, A.rcol, A.rval, w);
-        C.b[i] = bc;
-        C.r[i] = bc;
-      }
-    }
-    for (int i = threadIdx.x; i < n; i += kFuseThreads) uA[i] = x[i];
-    return;
   }
-  int nch = (C.n + kCoarseChunk - 1) / kCoarseChunk;
-  for (int i = threadIdx.x; i < C.n; i += kFuseThreads) w[i] = static_cast<T>(0) + coarse_sum(C.n, nch, i, part);
+  __device__ __forceinline__ int row(int i) const { return (ix[i].w >> 16) & 0xfff; }
+  __device__ __forceinline__ int color(int i) const { return ix[i].w >> 28; }
+  __device__ __forceinline__ int slot(int i, int k) const {
+    unsigned int w = k < 2 ? ix[i].x : k < 4 ? ix[i].y : k < 6 ? ix[i].z : ix[i].w;
+    w = opaque(w);
+    return (k & 1 ? w >> 16 : w) & 0xfff;
+  }
+  // b in w, a barrier behind it
+  __device__ __forceinline__ void rhs(const T *w) {
+#pragma unroll
+    for (int i = 0; i < R; i++) b[i] = w[row(i)];
+  }
+  __device__ __forceinline__ void sweep(T *x, int ncolors, bool reverse) {
+    for (int ci = 0; ci < ncolors; ci++) {
+      int c = reverse ? ncolors - 1 - ci : ci;
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        if (color(i) != c) continue;
+        T xs[S], sum = static_cast<T>(0);
+#pragma unroll
+        for (int k = 0; k < S; k++) xs[k] = x[slot(i, k)];
+#pragma unroll
+        for (int k = 0; k < S; k++) sum = sum + off[i][k] * xs[k];
+        x[row(i)] = (b[i] - sum) / d[i];
+      }
+      __syncthreads();
+    }
+  }
+};
+
+template <int S, class T, int R>
+__global__ void __launch_bounds__(kFuseThreads)
+    k_tail_down(const Tail<T> A, const T *__restrict__ u, const T *__restrict__ b, T *__restrict__ us,
+                T *__restrict__ z, int steps) {
+  constexpr int kGroups = kFuseThreads / kTailZ, kZ = 16;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int n = A.n, nc = A.nc, tid = threadIdx.x;
+  T *x = reinterpret_cast<T *>(smem_raw), *w = x + tail_x(n, nc), *rl = w + n;
+  TailRows<S, T, R> o;
+  o.load(A);
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    int r = tid + i * kFuseThreads;
+    if (r < n) {
+      x[r] = u ? u[r] : static_cast<T>(0);
+      w[r] = b[r];
+    }
+  }
   __syncthreads();
-  for (int j = threadIdx.x; j < n; j += kFuseThreads)
-    x[j] = uA[j] + (A.pwidth == 2 ? dec_ell::row<2, T, T>(n, A.pwidth, j, A.pcol, A.pval, w)
-                                  : dec_ell::row<0, T, T>(n, A.pwidth, j, A.pcol, A.pval, w));
+  o.rhs(w);
   __syncthreads();
-  for (int it = 0; it < steps; it++) sweep_owned<W, T, R>(o, x, 0, n, A.ncolors, true);
-  for (int i = threadIdx.x; i < n; i += kFuseThreads) uA[i] = x[i];
+  for (int it = 0; it < steps; it++) o.sweep(x, A.ncolors, false);
+  // the thread's first half chunk of a row of Z and its row of the restriction,
+  // on their way while the residual is formed
+  const int zi = blockIdx.x * kTailZ + tid % kTailZ, g = tid / kTailZ, j0 = g * kZ;
+  const bool direct = A.ZT != nullptr, zrow = direct && zi < nc;
+  T zt[kZ];
+  auto zload = [&](int k0, int k1) {
+#pragma unroll
+    for (int k = 0; k < kZ; k++)
+      if (k >= k0 && k < k1)
+        zt[k] = zrow && j0 + k < nc ? A.ZT[static_cast<size_t>(j0 + k) * nc + zi] : static_cast<T>(0);
+  };
+  zload(0, kZ / 2);
+  const bool pre = A.rwidth <= 8 && tid < nc;
+  int rc[8];
+  T rv[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    rc[k] = -1;
+    rv[k] = static_cast<T>(0);
+    if (pre && k < A.rwidth) {
+      rc[k] = A.rcol[static_cast<size_t>(k) * nc + tid];
+      rv[k] = A.rval[static_cast<size_t>(k) * nc + tid];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    if (o.color(i) == 15) continue;
+    int at = (o.ix[i].x >> 12) & 0xf;
+    T acc = static_cast<T>(0), dx = o.d[i] * x[o.row(i)];
+#pragma unroll
+    for (int k = 0; k < S; k++) {
+      if (k == at) acc = acc + dx;
+      acc = acc + o.off[i][k] * x[o.slot(i, k)];
+    }
+    if (at >= S) acc = acc + dx;
+    w[o.row(i)] = o.b[i] - acc;
+  }
+  zload(kZ / 2, kZ);
+  for (int r = blockIdx.x * kFuseThreads + tid; r < n; r += static_cast<int>(gridDim.x) * kFuseThreads) us[r] = x[r];
+  __syncthreads();
+  for (int i = tid; i < nc; i += kFuseThreads) {
+    T acc = static_cast<T>(0);
+    if (i == tid && pre) {
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (rc[k] >= 0) acc = acc + rv[k] * w[rc[k]];
+    } else {
+      acc = dec_ell::row<0, T, T>(nc, A.rwidth, i, A.rcol, A.rval, w);
+    }
+    if (direct) rl[i] = acc;
+    else z[i] = acc;
+  }
+  if (!direct) return;
+  __syncthreads();
+  const int nch = coarse_chunks(nc);
+  if (zrow && g < nch) {
+    T acc = static_cast<T>(0);
+#pragma unroll
+    for (int k = 0; k < kZ; k++)
+      if (j0 + k < nc) acc = acc + zt[k] * rl[j0 + k];
+    x[g * kTailZ + tid % kTailZ] = acc;
+    for (int c = g + kGroups; c < nch; c += kGroups) {
+      acc = static_cast<T>(0);
+#pragma unroll 8
+      for (int j = c * kZ; j < min(nc, (c + 1) * kZ); j++) acc = acc + A.ZT[static_cast<size_t>(j) * nc + zi] * rl[j];
+      x[c * kTailZ + tid % kTailZ] = acc;
+    }
+  }
+  __syncthreads();
+  if (tid < kTailZ && zrow) {
+    T t = static_cast<T>(0);
+#pragma unroll 8
+    for (int c = 0; c < nch; c++) t = t + x[c * kTailZ + tid];
+    z[zi] = t;
+  }
+}
+
+template <int S, class T, int R>
+__global__ void __launch_bounds__(kFuseThreads)
+    k_tail_up(const Tail<T> A, const T *__restrict__ us, const T *__restrict__ z, const T *__restrict__ b,
+              T *__restrict__ u, int steps) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int n = A.n, nc = A.nc, tid = threadIdx.x;
+  T *x = reinterpret_cast<T *>(smem_raw), *w = x + tail_x(n, nc), *rl = w + n;
+  TailRows<S, T, R> o;
+  int pc[R][2];
+  T pv[R][2], ur[R];
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    int r = tid + i * kFuseThreads, rc = min(r, n - 1);
+    ur[i] = us[rc];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      pc[i][k] = A.pwidth == 2 ? A.pcol[static_cast<size_t>(k) * n + rc] : -1;
+      pv[i][k] = A.pwidth == 2 ? A.pval[static_cast<size_t>(k) * n + rc] : static_cast<T>(0);
+    }
+    if (r < n) w[r] = b[r];
+  }
+  for (int i = tid; i < nc; i += kFuseThreads) rl[i] = z[i];
+  o.load(A);
+  __syncthreads();
+  o.rhs(w);
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    int r = tid + i * kFuseThreads;
+    if (r >= n) continue;
+    T acc = static_cast<T>(0);
+    if (A.pwidth == 2) {
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+        if (pc[i][k] >= 0) acc = acc + pv[i][k] * rl[pc[i][k]];
+    } else {
+      acc = dec_ell::row<0, T, T>(n, A.pwidth, r, A.pcol, A.pval, rl);
+    }
+    x[r] = ur[i] + acc;
+  }
+  __syncthreads();
+  for (int it = 0; it < steps; it++) o.sweep(x, A.ncolors, true);
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    int r = tid + i * kFuseThreads;
+    if (r < n) u[r] = x[r];
+  }
 }
 
 // ---------------------------------------------------------------- storage
@@ -1755,6 +1888,7 @@ struct LevelVals {
   DBuf<T> pval;  // ELL values of P (next coarser -> this level)
   DBuf<T> poff, pdiag;  // values of the Gauss-Seidel panels (k_panel_sweep)
   DBuf<T> pown_w, phalo_w;  // and P's values, two per row and per halo row
+  DBuf<T> toff, tdiag;  // values of the coarse tail's rows (Tail)
   DBuf<T> Z;     // dense coarse operator, column-major (coarsest level, direct solve)
   DBuf<T> zpart; // chunk partial products of the direct solve (coarsest level)
   DBuf<T> u, b, r, t;  // work vectors
@@ -1796,6 +1930,7 @@ struct Level {
   int panel_b = 0, panel_full = 0, panel_hs = -1;
   DBuf<uint32_t> pidx;
   DBuf<int32_t> phalo, pown_p, phalo_p;
+  DBuf<uint32_t> tidx;  // the coarse tail's rows (empty: not one), see Tail
 };
 
 }  // namespace
@@ -2040,6 +2175,32 @@ void build_panels(Level &L, const std::vector<int32_t> &color) {
   to_float(L.d.poff, L.f.poff);
   to_float(L.d.pdiag, L.f.pdiag);
   dec::check_launch("multigrid panels");
+}
+
+// The rows of the coarse tail (see Tail) of a level that can be one: every row
+// with a diagonal, at most 7 other entries, and vectors that fit in 64 KiB of LDS.
+void build_tail(Level &L, const LevelDesc<double> &D) {
+  const int n = L.n, S = std::max(L.width - 1, 1);
+  if (n < 1 || n > kTailRows || L.width < 1 || L.width > 8 || L.ncolors > 15 || L.nc < 1 ||
+      coarse_chunk(L.nc) != 16 || tail_lds(n, L.nc, sizeof(double)) > 64 * 1024)
+    return;
+  for (int r = 0; r < n; r++) {
+    int diag = 0;
+    for (int q = L.A.ptr[r]; q < L.A.ptr[r + 1]; q++) diag += L.A.col[q] == r;
+    if (diag != 1 || L.A.ptr[r + 1] - L.A.ptr[r] - 1 > S) return;
+  }
+  L.tidx.alloc(4 * static_cast<size_t>(n));
+  L.d.toff.alloc(static_cast<size_t>(S) * n);
+  L.d.tdiag.alloc(n);
+  hipLaunchKernelGGL(k_build_tail, dim3(dec::nblocks(n)), dim3(256), 0, 0, D, S, reinterpret_cast<uint4 *>(L.tidx.p),
+                     L.d.toff.p, L.d.tdiag.p);
+  auto to_float = [](const DBuf<double> &x, DBuf<float> &y) {
+    y.alloc(x.n);
+    hipLaunchKernelGGL(k_to_float, dim3(dec::nblocks(static_cast<long long>(x.n))), dim3(256), 0, 0, x.n, x.p, y.p);
+  };
+  to_float(L.d.toff, L.f.toff);
+  to_float(L.d.tdiag, L.f.tdiag);
+  dec::check_launch("multigrid tail");
 }
 
 // P's rows (width 2) of a level's own rows and of its panels' halos, for the
@@ -2387,6 +2548,7 @@ void finish_hierarchy(dec_mg_s &mg, const std::vector<dec::HostCsr> &As, std::ve
     mg.hdesc64 = d64;
     mg.hdesc32 = d32;
   }
+  for (int l = 0; l + 1 < nl; l++) build_tail(*mg.lv[l], mg.hdesc64[l]);
   mg.part.alloc(4 * kCgBlocksMax);  // also the dot partials (kDotBlocks of them)
   mg.part2.alloc(4 * kCgBlocksMax);
   mg.scal.alloc(8);
@@ -2791,6 +2953,45 @@ void coarse_solve(dec_mg_s &mg, Level &L, const T *b, T *u, hipStream_t s) {
 }
 
 // _multigrid_μ_cycle (Multigrid.jl:857-872).
+// The coarse tail's launch at level l, on the way down (C's solution, or above
+// the level before the last C's right-hand side, from b and u; the smoothed u goes to
+// the level's r) or up.
+template <class T>
+void tail_launch(dec_mg_s &mg, int l, const T *b, T *u, bool u_zero, bool up, hipStream_t s) {
+  Level &L = *mg.lv[l], &C = *mg.lv[l + 1];
+  LevelVals<T> &V = vals<T>(L), &CV = vals<T>(C);
+  const bool last = l + 2 == static_cast<int>(mg.lv.size());
+  Tail<T> A{L.n,      L.nc,      L.ncolors, L.rwidth, L.pwidth, reinterpret_cast<const uint4 *>(L.tidx.p),
+            V.toff.p, V.tdiag.p, L.rcol.p,  L.pcol.p, V.rval.p, V.pval.p,
+            last ? CV.Z.p : nullptr};
+  const size_t lds = tail_lds(L.n, L.nc, sizeof(T));
+  const dim3 grid(up || !last ? 1 : (L.nc + kTailZ - 1) / kTailZ), blk(kFuseThreads);
+  auto run = [&](auto S, auto R) {
+    if (up)
+      hipLaunchKernelGGL((k_tail_up<S.value, T, R.value>), grid, blk, lds, s, A, V.r.p, last ? CV.zpart.p : CV.u.p, b,
+                         u, mg.steps);
+    else
+      hipLaunchKernelGGL((k_tail_down<S.value, T, R.value>), grid, blk, lds, s, A,
+                         u_zero ? static_cast<const T *>(nullptr) : u, b, V.r.p, last ? CV.zpart.p : CV.b.p, mg.steps);
+  };
+  auto rows = [&](auto S) {
+    switch ((L.n + kFuseThreads - 1) / kFuseThreads) {
+      case 1: run(S, std::integral_constant<int, 1>{}); break;
+      case 2: run(S, std::integral_constant<int, 2>{}); break;
+      default: run(S, std::integral_constant<int, 3>{}); break;
+    }
+  };
+  switch (std::max(L.width - 1, 1)) {
+    case 1: rows(std::integral_constant<int, 1>{}); break;
+    case 2: rows(std::integral_constant<int, 2>{}); break;
+    case 3: rows(std::integral_constant<int, 3>{}); break;
+    case 4: rows(std::integral_constant<int, 4>{}); break;
+    case 5: rows(std::integral_constant<int, 5>{}); break;
+    case 6: rows(std::integral_constant<int, 6>{}); break;
+    default: rows(std::integral_constant<int, 7>{}); break;
+  }
+}
+
 template <class T>
 void mu_cycle(dec_mg_s &mg, int lvl, T *u, const T *b, int mu, bool u_zero, hipStream_t s) {
   int nl = static_cast<int>(mg.lv.size());
@@ -2809,27 +3010,16 @@ void mu_cycle(dec_mg_s &mg, int lvl, T *u, const T *b, int mu, bool u_zero, hipS
       return;
     }
     Level &C = *mg.lv.back();
-    // one Gauss-Seidel level above the dense coarsest level: the register/LDS tail
-    if (lvl == nl - 2 && mg.alg != DEC_SMOOTH_JACOBI && L.n <= 3 * kFuseThreads && L.width >= 1 && L.width <= 8 &&
-        static_cast<size_t>(L.n + std::max(L.n, C.n)) * sizeof(T) <= 64 * 1024) {
-      size_t lds = static_cast<size_t>(L.n + std::max(L.n, C.n)) * sizeof(T);
-      const T *zp = vals<T>(C).zpart.p;
-      const std::vector<LevelDesc<T>> &HD = host_desc<T>(mg);
-      auto tail = [&](int phase) {
-        switch (L.width) {
-#define DEC_TAIL2(WW)                                                                                                 \
-  case WW:                                                                                                           \
-    hipLaunchKernelGGL((k_tail2<WW, T, 3>), dim3(1), dim3(kFuseThreads), lds, s, HD[lvl], HD[lvl + 1], u, b,       \
-                       mg.steps, phase, zp);                                                                          \
-    break;
-          DEC_TAIL2(1) DEC_TAIL2(2) DEC_TAIL2(3) DEC_TAIL2(4) DEC_TAIL2(5) DEC_TAIL2(6) DEC_TAIL2(7) DEC_TAIL2(8)
-#undef DEC_TAIL2
-          default: break;
-        }
-      };
-      tail(1);
-      coarse_partials<T>(C, s);
-      tail(2);
+    // Gauss-Seidel levels above the dense coarsest level: the register/LDS tail
+    bool tail = lvl < nl - 1 && mg.alg != DEC_SMOOTH_JACOBI;
+    for (int l = lvl; l < nl - 1; l++) tail = tail && mg.lv[l]->tidx.p;
+    if (tail) {
+      for (int l = lvl; l < nl - 1; l++)
+        tail_launch<T>(mg, l, l > lvl ? vals<T>(*mg.lv[l]).b.p : b, l > lvl ? vals<T>(*mg.lv[l]).u.p : u,
+                       l > lvl || u_zero, false, s);
+      for (int l = nl - 2; l >= lvl; l--)
+        tail_launch<T>(mg, l, l > lvl ? vals<T>(*mg.lv[l]).b.p : b, l > lvl ? vals<T>(*mg.lv[l]).u.p : u, false, true,
+                       s);
       return;
     }
     hipLaunchKernelGGL(k_fused_vcycle<T>, dim3(1), dim3(kFuseThreads), 0, s, D, lvl, nl, u, b, mg.steps, mg.alg, om,
