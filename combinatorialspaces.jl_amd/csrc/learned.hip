@@ -1197,11 +1197,11 @@ __global__ void k_hp_grad(int n, float scale, const float *__restrict__ eh, cons
 //
 // What bounds them: the h and dz rows read and written (0.46 GB at 16 x 40,962
 // rows, about 90 µs of HBM time) and the gathers' dependent loads.  Measured at
-// that size, loss and gradient of the error loss: 338 µs, against 2,020 µs with
+// that size, loss and gradient of the error loss: 289 µs, against 2,020 µs with
 // one kernel per operation (dg in FP32, two launches per reduction), the
 // gradient as far from its value in 64 bits as before (4.1e-3 of its norm).
 
-constexpr int kBackBlocks = 512;           // at most; a multiple of 8
+constexpr int kBackBlocks = 768;           // at most, three a CU; a multiple of 8
 constexpr int kBackPitch = 4 * H + 8;      // bf16 per LDS row: [dz | q high | q low | h] plus padding
 
 // x = r / s, P x and the layer-1 rows h1 (the values of k_input).
@@ -1459,14 +1459,12 @@ __global__ void __launch_bounds__(TB) k_head_back(int n, int B, int nc, int aw, 
   }
 }
 
-// four consecutive rows' entries of one LDS column, as an MFMA operand over rows
-__device__ __forceinline__ short4_t lds_col4(const unsigned short *p) {
-  short4_t a;
-  a[0] = static_cast<short>(p[0]);
-  a[1] = static_cast<short>(p[kBackPitch]);
-  a[2] = static_cast<short>(p[2 * kBackPitch]);
-  a[3] = static_cast<short>(p[3 * kBackPitch]);
-  return a;
+// Four consecutive rows' entries of one LDS column, as an MFMA operand over rows:
+// lane li of a group of 16 gets column li of the group's four rows (pitch
+// kBackPitch).  The read transposes: lane li reads columns 4 (li & 3) .. of row li >> 2.
+__device__ __forceinline__ short4_t lds_col4(unsigned short *rows, int li) {
+  typedef short4_t __attribute__((address_space(3))) * Lds;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(rows + (li >> 2) * kBackPitch + 4 * (li & 3)));
 }
 
 // One dense layer's backward step.  dz of the layer: HEAD, formed from dm (dy
@@ -1475,17 +1473,17 @@ __device__ __forceinline__ short4_t lds_col4(const unsigned short *p) {
 // g = dh ⊙ [hb > 0] at ob_below; HEAD: of dz at ob_self, and g is stored in BF16
 // as the dz of the layer below; else: of (x g, P x g) at OW1.
 template <int W, bool HEAD>
-__global__ void __launch_bounds__(TB)
+__global__ void __launch_bounds__(TB, 3)
     k_layer_back(int n, int B, const int *__restrict__ ptcol, const float *__restrict__ ptval,
                  const unsigned short *__restrict__ dzin, const float2 *__restrict__ dm, const float *__restrict__ wo,
                  const unsigned short *__restrict__ hb, const float *__restrict__ Wt, unsigned short *__restrict__ dzout,
                  const float *__restrict__ x, const float *__restrict__ px, float *__restrict__ part_out, int ow,
                  int ob_below, int ob_self) {
-  __shared__ __align__(16) unsigned short rows_s[kInfWaves][64 * kBackPitch];
+  __shared__ __align__(16) unsigned short rows_s[kInfWaves][2][16 * kBackPitch];
   __shared__ float2 xs_s[HEAD ? 1 : kInfWaves][64];
+  static_assert(sizeof(rows_s) >= kInfWaves * 32 * 64 * sizeof(float), "the sums at the end");
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4, sub = lane >> 2, part = lane & 3;
-  unsigned short *rows = rows_s[wv];
   const int T = (n + 63) / 64;
   // Wᵀ as B operands: own rows of W and neighbour rows
   short4_t Bo[2][2], Bn[2][2];
@@ -1514,36 +1512,50 @@ __global__ void __launch_bounds__(TB)
   for (int e = 0; e < 8; e++) osum[e] = 0.0f;
   int wt, wend, step;
   wave_tiles(B * T, wt, wend, step);
+  // One 16-row group at a time, four to a tile: the rows pass through 8.7 KB of
+  // LDS a wavefront, so that three workgroups fit in a CU by their registers (64
+  // rows at once: 17 KB, two workgroups), and the groups are not unrolled, which
+  // keeps their addresses out of registers.  16 x 40,962 rows, HEAD and not: 63
+  // and 70 µs with 64 rows at once and columns read entry by entry, 56 and
+  // 38 so; with the next group's gathers issued ahead of the products, two
+  // workgroups a CU, 58 and 41; held to four, with spills, 61 and 42.
+  int c[W];
+  float pv[W];
   for (; wt < wend; wt += step) {
-    int b = wt / T, t = wt - b * T;
+    const int b = wt / T, t = wt - b * T;
     const size_t o = static_cast<size_t>(b) * n;
-    int c[W];
-    float pv[W];
     own_slots<W>(n, t * 64 + lane, ptcol, ptval, c, pv);
     if constexpr (!HEAD) {
-      int vv = min(t * 64 + lane, n - 1);
-      xs_s[wv][lane] = make_float2(x[o + vv], px[o + vv]);
+      size_t i = o + min(t * 64 + lane, n - 1);
+      xs_s[wv][lane] = make_float2(x[i], px[i]);
     }
-#pragma unroll
+#pragma unroll 1
     for (int g = 0; g < 4; g++) {
-      int r = t * 64 + 16 * g + sub;
-      size_t rr = o + min(r, n - 1);
-      int cg[W];
-      float vg[W];
+      unsigned short *rows = rows_s[wv][g & 1];
+      const int r = t * 64 + 16 * g + sub;
+      const size_t rr = o + min(r, n - 1);
+      uint4 hr, own, a[HEAD ? 1 : W];
+      float2 od, nd[HEAD ? W : 1];
+      hr = *reinterpret_cast<const uint4 *>(hb + rr * H + 8 * part);
+      if constexpr (HEAD) od = dm[rr];
+      else own = *reinterpret_cast<const uint4 *>(dzin + rr * H + 8 * part);
+      unsigned int have = 0;  // the row's slots that are not pads
 #pragma unroll
       for (int k = 0; k < W; k++) {
-        cg[k] = __shfl(c[k], 16 * g + sub);
-        vg[k] = __shfl(pv[k], 16 * g + sub);
+        int cg = __shfl(c[k], 16 * g + sub);
+        have |= (cg >= 0 ? 1u : 0u) << k;
+        size_t i = o + (cg < 0 ? 0 : cg);
+        if constexpr (HEAD) nd[k] = dm[i];
+        else a[k] = *reinterpret_cast<const uint4 *>(dzin + i * H + 8 * part);
       }
-      uint4 hr = *reinterpret_cast<const uint4 *>(hb + rr * H + 8 * part);
       float q[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) q[e] = 0.0f;
-      uint4 own;
-      if constexpr (HEAD) {
-        float2 od = dm[rr], nd[W];
+      float vg[W];
 #pragma unroll
-        for (int k = 0; k < W; k++) nd[k] = dm[o + (cg[k] < 0 ? 0 : cg[k])];
+      for (int k = 0; k < W; k++) vg[k] = __shfl(pv[k], 16 * g + sub);
+      uint4 mine;
+      if constexpr (HEAD) {
         auto form = [&](float2 d, bool keep) {
           unsigned int m = keep ? __float_as_uint(d.y) >> (8 * part) : 0u;
           float z[8];
@@ -1551,28 +1563,23 @@ __global__ void __launch_bounds__(TB)
           for (int e = 0; e < 8; e++) z[e] = (m >> e) & 1u ? d.x * wl[e] : 0.0f;
           return pack8(z);
         };
-        own = form(od, r < n);
+        mine = form(od, r < n);
         float f[8];
-        unpack8(own, f);
+        unpack8(mine, f);
 #pragma unroll
         for (int e = 0; e < 8; e++) osum[e] += f[e];
 #pragma unroll
         for (int k = 0; k < W; k++) {
-          unpack8(form(nd[k], cg[k] >= 0), f);
+          unpack8(form(nd[k], have >> k & 1u), f);
 #pragma unroll
           for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
         }
       } else {
-        own = keep_if(*reinterpret_cast<const uint4 *>(dzin + rr * H + 8 * part), r < n);
-        uint4 a[W];
-#pragma unroll
-        for (int k = 0; k < W; k++)
-          a[k] = keep_if(*reinterpret_cast<const uint4 *>(dzin + (o + (cg[k] < 0 ? 0 : cg[k])) * H + 8 * part),
-                         cg[k] >= 0);
+        mine = keep_if(own, r < n);
 #pragma unroll
         for (int k = 0; k < W; k++) {
           float f[8];
-          unpack8(a[k], f);
+          unpack8(keep_if(a[k], have >> k & 1u), f);
 #pragma unroll
           for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
         }
@@ -1582,24 +1589,21 @@ __global__ void __launch_bounds__(TB)
       unpack8(hi, fh);
 #pragma unroll
       for (int e = 0; e < 8; e++) q[e] = q[e] - fh[e];
-      unsigned short *d = rows + (16 * g + sub) * kBackPitch + 8 * part;
-      *reinterpret_cast<uint4 *>(d) = own;
+      unsigned short *d = rows + sub * kBackPitch + 8 * part;
+      *reinterpret_cast<uint4 *>(d) = mine;
       *reinterpret_cast<uint4 *>(d + H) = hi;
       *reinterpret_cast<uint4 *>(d + 2 * H) = pack8(q);
       *reinterpret_cast<uint4 *>(d + 3 * H) = keep_if(hr, r < n);
-    }
-    wave_sync();
-    // dW += hᵀ dz, hᵀ q: four steps of 16 rows
-#pragma unroll
-    for (int ks = 0; ks < 4; ks++) {
-      const unsigned short *base = rows + (16 * ks + 4 * lg) * kBackPitch + li;
+      wave_sync();
+      // dW += hᵀ dz, hᵀ q
+      unsigned short *base = rows + 4 * lg * kBackPitch;
       short4_t A[2], Z[2], Q[2], L[2];
 #pragma unroll
       for (int k = 0; k < 2; k++) {
-        A[k] = lds_col4(base + 3 * H + 16 * k);
-        Z[k] = lds_col4(base + 16 * k);
-        Q[k] = lds_col4(base + H + 16 * k);
-        L[k] = lds_col4(base + 2 * H + 16 * k);
+        A[k] = lds_col4(base + 3 * H + 16 * k, li);
+        Z[k] = lds_col4(base + 16 * k, li);
+        Q[k] = lds_col4(base + H + 16 * k, li);
+        L[k] = lds_col4(base + 2 * H + 16 * k, li);
       }
 #pragma unroll
       for (int ft = 0; ft < 2; ft++)
@@ -1609,49 +1613,41 @@ __global__ void __launch_bounds__(TB)
           aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], Q[jt], aN[ft][jt], 0, 0, 0);
           aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], L[jt], aN[ft][jt], 0, 0, 0);
         }
-    }
-    // dh of 16 rows at a time, masked by the signs of h
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-      const unsigned short *rp = rows + (16 * g + li) * kBackPitch + 4 * lg;
-      short4_t Z[2] = {lds4(rp), lds4(rp + 16)}, Q[2] = {lds4(rp + H), lds4(rp + H + 16)},
-               L[2] = {lds4(rp + 2 * H), lds4(rp + 2 * H + 16)};
+      // dh, masked by the signs of h
+      const unsigned short *rp = rows + li * kBackPitch + 4 * lg;
+      short4_t Zr[2] = {lds4(rp), lds4(rp + 16)}, Qr[2] = {lds4(rp + H), lds4(rp + H + 16)},
+               Lr[2] = {lds4(rp + 2 * H), lds4(rp + 2 * H + 16)};
+      wave_sync();
 #pragma unroll
       for (int jt = 0; jt < 2; jt++) {
-        float4_t a = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
-          a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Z[ks], Bo[jt][ks], a, 0, 0, 0);
-          a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(L[ks], Bn[jt][ks], a, 0, 0, 0);
-          a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Q[ks], Bn[jt][ks], a, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Zr[ks], Bo[jt][ks], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Lr[ks], Bn[jt][ks], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Qr[ks], Bn[jt][ks], acc, 0, 0, 0);
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          int row = 16 * g + 4 * lg + i;
-          unsigned short *d = rows + row * kBackPitch;
-          // h is zero in rows past the end, so those add nothing
-          float gv = bf2f(d[3 * H + 16 * jt + li]) > 0.0f ? a[i] : 0.0f;
+          // h is zero in rows past the end, so those add nothing; A holds h of
+          // the accumulator's own rows and column
+          float gv = bf2f(static_cast<unsigned short>(A[jt][i])) > 0.0f ? acc[i] : 0.0f;
           bsum[jt] += gv;
           if constexpr (HEAD) {
-            d[16 * jt + li] = f2bf(gv);
+            rows[(4 * lg + i) * kBackPitch + 16 * jt + li] = f2bf(gv);
           } else {
-            float2 xp = xs_s[wv][row];
+            float2 xp = xs_s[wv][16 * g + 4 * lg + i];
             w1[jt] += xp.x * gv;
             w1[2 + jt] += xp.y * gv;
           }
         }
       }
-    }
-    wave_sync();
-    if constexpr (HEAD) {
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        int r = t * 64 + 16 * g + sub;
+      if constexpr (HEAD) {
+        wave_sync();
         if (r < n)
           *reinterpret_cast<uint4 *>(dzout + (o + r) * H + 8 * part) =
-              *reinterpret_cast<const uint4 *>(rows + (16 * g + sub) * kBackPitch + 8 * part);
+              *reinterpret_cast<const uint4 *>(rows + sub * kBackPitch + 8 * part);
       }
-      wave_sync();
     }
   }
   // the wavefronts' sums into one row of partials
