@@ -49,7 +49,8 @@ __global__ void k_residual(int n, int width, const int *__restrict__ col, const 
   r[v] = b[v] - acc;
 }
 
-// The residual r = b - A u of k_residual and, per workgroup, the sum of its
+// The residual r = b - A u of k_residual (in float64, in float32 where a float32
+// cycle takes it, or both) and, per workgroup, the sum of its
 // rows' r² (a fixed tree) into part[blockIdx.x]; k_sum_rows adds the
 // partial sums.  (A ticket letting the last workgroup add them needs a
 // device-scope fence in every workgroup, which writes back the XCD's L2:
@@ -58,7 +59,7 @@ template <int W>
 __global__ void __launch_bounds__(256)
     k_residual_norm(int n, int width, const int *__restrict__ col, const double *__restrict__ val,
                     const int *__restrict__ rowid, const double *__restrict__ b, const double *__restrict__ u,
-                    double *__restrict__ r, double *__restrict__ part) {
+                    double *__restrict__ r, float *__restrict__ rf, double *__restrict__ part) {
   __shared__ double sh[256];
   int p = blockIdx.x * blockDim.x + threadIdx.x;
   double rr = 0.0;
@@ -66,7 +67,8 @@ __global__ void __launch_bounds__(256)
     double acc = dec_ell::row<W, double, double>(n, width, p, col, val, u);
     int v = rowid ? rowid[p] : p;
     double ri = b[v] - acc;
-    r[v] = ri;
+    if (r) r[v] = ri;
+    if (rf) rf[v] = static_cast<float>(ri);
     rr = ri * ri;
   }
   sh[threadIdx.x] = rr;
@@ -301,7 +303,8 @@ struct Vec2T<float> {
 // loads: they take two round trips (rows, vectors and halo numbers; the halo's
 // values).  ZERO: u is zero on entry and is not read.  zc: the sweep starts from
 // u + P zc (P of width 2, also for the halo).  dot (when given): the block's Σ b u
-// after the sweep.  Per-row arithmetic is k_block_gs's, bit for bit.
+// after the sweep.  add (float32, when given): the swept u is added to it
+// and not stored.  Per-row arithmetic is k_block_gs's, bit for bit.
 // Measured (µs a sweep, float64, levels 3->8): 655,362 rows 14.4 (11.6 from zero;
 // bound by bytes: 3.9 TB/s), against 18.2 with the colours' rows streamed one
 // after the other; below 200,000 rows 4.7 (4.1 from zero; bound by the two round
@@ -321,7 +324,7 @@ struct Panels {
 template <int W, class T, int R, bool ZERO>
 __global__ void __launch_bounds__(256)
     k_panel_sweep(Panels<T> P, const T *__restrict__ b, const T *__restrict__ uin, T *__restrict__ uout, int reverse,
-                  const T *__restrict__ zc, double *__restrict__ dot) {
+                  const T *__restrict__ zc, double *__restrict__ dot, double *__restrict__ add) {
   constexpr int S = W - 1;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *x = reinterpret_cast<T *>(smem_raw), *bl = x + P.B + P.hs;
@@ -417,6 +420,12 @@ __global__ void __launch_bounds__(256)
     row[m] = static_cast<int>(w & 0xfffu);
     bv[m] = bl[row[m]];
   }
+  double added[R];  // what the sweep's result is added to, on its way during the colours
+#pragma unroll
+  for (int m = 0; m < R; m++) {
+    int i = t + m * nt;
+    added[m] = sizeof(T) == 4 && add && i < nr ? add[r0 + i] : 0.0;
+  }
   for (int ci = 0; ci < P.ncolors; ci++) {
     int c = reverse ? P.ncolors - 1 - ci : ci;
 #pragma unroll
@@ -439,7 +448,8 @@ __global__ void __launch_bounds__(256)
     int i = t + m * nt;
     if (i < nr) {
       T v = x[i];
-      uout[r0 + i] = v;
+      if (sizeof(T) == 4 && add) add[r0 + i] = added[m] + static_cast<double>(v);
+      else uout[r0 + i] = v;
       acc = acc + static_cast<double>(bl[i]) * static_cast<double>(v);
     }
   }
@@ -1355,11 +1365,6 @@ __global__ void __launch_bounds__(kCgThreads)
   }
 }
 
-__global__ void k_d2f(int n, const double *__restrict__ x, float *__restrict__ y) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = static_cast<float>(x[i]);
-}
-
 __global__ void k_add_f2d(int n, const float *__restrict__ c, double *__restrict__ u) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) u[i] = u[i] + static_cast<double>(c[i]);
@@ -1967,6 +1972,7 @@ struct dec_mg_s {
   // where the finest level's last post-sweep puts its blocks' sums of b u
   // (set while a preconditioned-CG iteration is queued, else null)
   double *sweep_dot = nullptr;
+  double *sweep_add = nullptr;  // the float64 iterate that takes the finest level's last float32 sweep
   // residual norms of a solve on their way to the host (pinned ring + events)
   DBuf<double> rpart;  // per-workgroup partial sums of the finest residual's r²
   // (slot kNormSlots: ||b||^2 of the solve)
@@ -2823,7 +2829,7 @@ constexpr int kCgFoldMaxRows = 100000;
 // One panel sweep (k_panel_sweep) from src (zero: src is zero and not read) to dst.
 template <class T>
 void panel_sweep(Level &L, const T *b, const T *src, T *dst, bool post, bool zero, const T *zc, double *dot,
-                 hipStream_t s) {
+                 double *add, hipStream_t s) {
   LevelVals<T> &V = vals<T>(L);
   using V2 = typename Vec2T<T>::type;
   Panels<T> P{L.panel_b,
@@ -2843,7 +2849,7 @@ void panel_sweep(Level &L, const T *b, const T *src, T *dst, bool post, bool zer
   size_t lds = static_cast<size_t>(2 * P.B + P.hs) * sizeof(T);
   int rev = post ? 1 : 0;
 #define DEC_PANEL(WW, RR, ZZ) \
-  hipLaunchKernelGGL((k_panel_sweep<WW, T, RR, ZZ>), dim3(L.nblk), dim3(nt), lds, s, P, b, src, dst, rev, zc, dot)
+  hipLaunchKernelGGL((k_panel_sweep<WW, T, RR, ZZ>), dim3(L.nblk), dim3(nt), lds, s, P, b, src, dst, rev, zc, dot, add)
 #define DEC_PANEL_W(WW)                      \
   case WW:                                   \
     if (P.B <= kBlock) {                     \
@@ -2901,13 +2907,15 @@ void smooth(dec_mg_s &mg, int lvl, Level &L, const T *b, T *u, bool post, bool u
       T *dst = bufs[(it + 1) & 1];
       if (L.panel_hs >= 0)
         panel_sweep<T>(L, b, src, dst, post, u_zero && it == 0, it == 0 ? zc : nullptr,
-                       post && lvl == 0 && it + 1 == steps ? mg.sweep_dot : nullptr, s);
+                       post && lvl == 0 && it + 1 == steps ? mg.sweep_dot : nullptr,
+                       post && lvl == 0 && it + 1 == steps ? mg.sweep_add : nullptr, s);
       else
         DEC_ELL_WIDTH_SWITCH(L.width, hipLaunchKernelGGL((k_block_gs<W, T>), dim3(L.nblk), dim3(L.seg_threads), lds,
                                                          s, L.n, L.width, L.ncolors, L.nblk, L.col.p, V.val.p,
                                                          L.rowid.p, L.bstart.p, L.seg.p, b, src, dst, post ? 1 : 0));
     }
-    if (steps & 1) hipLaunchKernelGGL(k_copy<T>, G(L.n), dim3(kBlock), 0, s, L.n, V.t.p, u);
+    if (steps & 1 && !(post && lvl == 0 && mg.sweep_add))
+      hipLaunchKernelGGL(k_copy<T>, G(L.n), dim3(kBlock), 0, s, L.n, V.t.p, u);
     return;
   }
   for (int it = 0; it < steps; it++) {
@@ -3138,11 +3146,15 @@ void cycle_body(dec_mg_s &mg, int variant, double *u, const double *b, hipStream
   if (variant == DEC_SOLVE_PLAIN_F64) {
     mu_cycle<double>(mg, 0, u, b, 1, false, s);
   } else {
-    // float32 V-cycle on the float64 residual, correction added in float64
-    hipLaunchKernelGGL(k_d2f, G(n), dim3(kBlock), 0, s, n, F.d.r.p, F.f.b.p);
-    if (!zero_unread<float>(mg, F)) hipLaunchKernelGGL(k_zero<float>, G(n), dim3(kBlock), 0, s, n, F.f.u.p);
+    // float32 V-cycle on the float64 residual (rounded by the launch that formed
+    // it), correction added in float64: by the cycle's last sweep where it is a
+    // panel sweep, which saves a launch (2.3 µs at 100,000 rows)
+    bool swept = zero_unread<float>(mg, F);
+    if (!swept) hipLaunchKernelGGL(k_zero<float>, G(n), dim3(kBlock), 0, s, n, F.f.u.p);
+    mg.sweep_add = swept ? u : nullptr;
     mu_cycle<float>(mg, 0, F.f.u.p, F.f.b.p, 1, true, s);
-    hipLaunchKernelGGL(k_add_f2d, G(n), dim3(kBlock), 0, s, n, F.f.u.p, u);
+    mg.sweep_add = nullptr;
+    if (!swept) hipLaunchKernelGGL(k_add_f2d, G(n), dim3(kBlock), 0, s, n, F.f.u.p, u);
   }
 }
 
@@ -3250,7 +3262,8 @@ void solve(dec_mg_s &mg, int variant, double tol, int max_cycles, double *u_call
     if (mg.rpart.n < static_cast<size_t>(nb)) fail(DEC_ERR_ARG, "multigrid: residual partials");
     DEC_ELL_WIDTH_SWITCH(F.width, hipLaunchKernelGGL((k_residual_norm<W>), dim3(nb), dim3(kBlock), 0, s, n, F.width,
                                                      F.vcol.p, F.d.vval.p, static_cast<const int *>(nullptr), b, u,
-                                                     F.d.r.p, mg.rpart.p));
+                                                     static_cast<double *>(nullptr), plain ? nullptr : F.f.b.p,
+                                                     mg.rpart.p));
     if (!check) return;
     double *slot = mg.scal.p + (k % kNormSlots);
     hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(kBlock), 0, s, nb, mg.rpart.p, slot);
@@ -3430,7 +3443,7 @@ void pcg_solve(dec_mg_s &mg, bool mixed, double tol, int max_iters, double *u_ca
   auto true_residual = [&](int k) {
     DEC_ELL_WIDTH_SWITCH(F.width, hipLaunchKernelGGL((k_residual_norm<W>), dim3(nb), dim3(kBlock), 0, s, n, F.width,
                                                      F.vcol.p, F.d.vval.p, static_cast<const int *>(nullptr), b, x,
-                                                     F.d.r.p, mg.rpart.p));
+                                                     F.d.r.p, static_cast<float *>(nullptr), mg.rpart.p));
     send(k, mg.rpart.p, nb);
   };
   // CG from the true residual in F.d.r
