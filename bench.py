@@ -628,12 +628,12 @@ def heat_instances(torch, cs, ninst=64, seed=7):
 
 def heat_step_bytes(levels, s):
     """Algorithmic bytes of one batched step: each instance's Laplacian rows
-    (nnz = nv + 2 ne entries of int32 column + value) and its state read and
-    written once."""
+    (16 bytes of packed columns a row, nnz = nv + 2 ne values) and its state
+    read and written once."""
     total = 0
     for k in levels:
         nv, ne = 10 * 4 ** k + 2, 30 * 4 ** k
-        total += (nv + 2 * ne) * (4 + s) + 2 * nv * s
+        total += 16 * nv + (nv + 2 * ne) * s + 2 * nv * s
     return total
 
 
@@ -642,7 +642,7 @@ def batched_heat(torch, cs, ninst=64, nsteps=100, seed=7, counters=True):
     icosphere levels 4-7 (one mesh per instance), FP32, in one persistent
     launch per step replayed from a hipGraph, launch shape from the autotuner;
     checked against the same steps in FP64.  The working set (tables and
-    state, about 104 MB) fits the 256 MB Infinity Cache, so across steps the
+    state, about 75 MB) fits the 256 MB Infinity Cache, so across steps the
     tables come back from that cache: the rate is of L2-miss traffic, and the
     counter pass gives the bytes the L2 actually fetched and wrote."""
     levels, inst, b32, b64, u64 = heat_instances(torch, cs, ninst, seed)
