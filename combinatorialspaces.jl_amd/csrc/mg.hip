@@ -3144,6 +3144,16 @@ double norm2(dec_mg_s &mg, int n, const double *x, hipStream_t s) {
   return std::sqrt(v);
 }
 
+// What the finest level's last sweep also does, for one cycle (also where that
+// cycle ends with an exception).
+struct Hook {
+  double *&slot;
+  Hook(double *&s, double *p) : slot(s) { slot = p; }
+  ~Hook() { slot = nullptr; }
+  Hook(const Hook &) = delete;
+  Hook &operator=(const Hook &) = delete;
+};
+
 void cycle_body(dec_mg_s &mg, int variant, double *u, const double *b, hipStream_t s) {
   Level &F = *mg.lv[0];
   int n = F.n;
@@ -3155,9 +3165,10 @@ void cycle_body(dec_mg_s &mg, int variant, double *u, const double *b, hipStream
     // panel sweep, which saves a launch (2.3 µs at 100,000 rows)
     bool swept = zero_unread<float>(mg, F);
     if (!swept) hipLaunchKernelGGL(k_zero<float>, G(n), dim3(kBlock), 0, s, n, F.f.u.p);
-    mg.sweep_add = swept ? u : nullptr;
-    mu_cycle<float>(mg, 0, F.f.u.p, F.f.b.p, 1, true, s);
-    mg.sweep_add = nullptr;
+    {
+      Hook hook(mg.sweep_add, swept ? u : nullptr);
+      mu_cycle<float>(mg, 0, F.f.u.p, F.f.b.p, 1, true, s);
+    }
     if (!swept) hipLaunchKernelGGL(k_add_f2d, G(n), dim3(kBlock), 0, s, n, F.f.u.p, u);
   }
 }
@@ -3375,9 +3386,8 @@ void pcg_iteration(dec_mg_s &mg, bool mixed, double *x, hipStream_t s) {
   bool swept = !mixed && zero_unread<double>(mg, F);
   int np = swept ? F.nblk : kPcgDotBlocks;
   if (!mixed) {
-    mg.sweep_dot = swept ? part : nullptr;
+    Hook hook(mg.sweep_dot, swept ? part : nullptr);
     mu_cycle<double>(mg, 0, z, r, 1, true, s);
-    mg.sweep_dot = nullptr;
   } else {
     mu_cycle<float>(mg, 0, F.f.u.p, F.f.b.p, 1, true, s);
   }
