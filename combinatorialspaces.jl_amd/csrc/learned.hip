@@ -86,20 +86,21 @@ __device__ __forceinline__ float ell_row(int n, int width, int r, const int *__r
 // tree), summed in block order by one thread per sample.
 constexpr int kScaleBlocks = 128;
 
+template <int U>
 __global__ void k_scale_partial(int n, const float *__restrict__ r, double *__restrict__ part) {
   __shared__ double sh[TB];
   const float *rb = r + static_cast<size_t>(blockIdx.y) * n;
   double acc = 0.0;
   constexpr int stride = kScaleBlocks * TB;
-  // 32 loads in flight (one round trip up to 1,048,576 rows), added in the
-  // order of i; past the end a clamped load adds +0, which leaves the sum of
-  // squares unchanged
-  for (int i = blockIdx.x * TB + threadIdx.x; i < n; i += 32 * stride) {
-    float a[32];
+  // U loads in flight (one round trip up to 32,768 U rows; U fits n, see
+  // scale_partial), added in the order of i; past the end a clamped load adds +0, which
+  // leaves the sum of squares unchanged
+  for (int i = blockIdx.x * TB + threadIdx.x; i < n; i += U * stride) {
+    float a[U];
 #pragma unroll
-    for (int u = 0; u < 32; u++) a[u] = rb[min(i + u * stride, n - 1)];
+    for (int u = 0; u < U; u++) a[u] = rb[min(i + u * stride, n - 1)];
 #pragma unroll
-    for (int u = 0; u < 32; u++) acc += i + u * stride < n ? static_cast<double>(a[u]) * a[u] : 0.0;
+    for (int u = 0; u < U; u++) acc += i + u * stride < n ? static_cast<double>(a[u]) * a[u] : 0.0;
   }
   sh[threadIdx.x] = acc;
   __syncthreads();
@@ -108,6 +109,14 @@ __global__ void k_scale_partial(int n, const float *__restrict__ r, double *__re
     __syncthreads();
   }
   if (threadIdx.x == 0) part[static_cast<size_t>(blockIdx.y) * kScaleBlocks + blockIdx.x] = sh[0];
+}
+
+// A level of 40,962 rows needs two loads a thread, not 32 (16 samples: 8.1 to 3.8 µs).
+void scale_partial(int n, int B, const float *r, double *part, hipStream_t st) {
+  dim3 g(kScaleBlocks, B), blk(TB);
+  if (n <= 2 * kScaleBlocks * TB) hipLaunchKernelGGL(k_scale_partial<2>, g, blk, 0, st, n, r, part);
+  else if (n <= 8 * kScaleBlocks * TB) hipLaunchKernelGGL(k_scale_partial<8>, g, blk, 0, st, n, r, part);
+  else hipLaunchKernelGGL(k_scale_partial<32>, g, blk, 0, st, n, r, part);
 }
 
 __global__ void k_scale_final(int n, int B, const double *__restrict__ part, float *__restrict__ s) {
@@ -1119,21 +1128,22 @@ __global__ void k_loss(int n, int B, int aw, const int *__restrict__ acol, const
 
 // ---- error loss: mean (H ε)², ε = e / s - y / D, H = I - Pr R ---------------
 
+// Row i of an ELL times x: all loads of a row of at most 8 slots are issued at once
+// (R's and P's rows of a subdivided mesh: 16 x 10,242 rows of R 8.3 to 4.9 µs), wider rows
+// slot by slot; the same sum.
+__device__ __forceinline__ float row_of(int nrows, int width, int i, const int *__restrict__ col,
+                                        const float *__restrict__ val, const float *__restrict__ x) {
+  return width <= 8 ? dec_ell::row_upto<8, float, float>(nrows, width, i, col, val, x)
+                    : dec_ell::row<0, float, float>(nrows, width, i, col, val, x);
+}
+
 // y[b][i] = Σ_k val[k][i] x[b][col[k][i]] for a batch of vectors (rows ascending ELL)
 __global__ void k_bspmv(int nrows, int ncols, int width, const int *__restrict__ col, const float *__restrict__ val,
                         const float *__restrict__ x, float *__restrict__ y) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   int b = blockIdx.y;
   if (i >= nrows) return;
-  const float *xb = x + static_cast<size_t>(b) * ncols;
-  float acc = 0.0f;
-  for (int k = 0; k < width; k++) {
-    size_t q = static_cast<size_t>(k) * nrows + i;
-    int c = col[q];
-    if (c < 0) break;
-    acc = acc + val[q] * xb[c];
-  }
-  y[static_cast<size_t>(b) * nrows + i] = acc;
+  y[static_cast<size_t>(b) * nrows + i] = row_of(nrows, width, i, col, val, x + static_cast<size_t>(b) * ncols);
 }
 
 // eps = κ (e / s - y / D), κ = mean(D): the error in residual units
@@ -1197,7 +1207,7 @@ __global__ void k_hp_grad(int n, float scale, const float *__restrict__ eh, cons
 //
 // What bounds them: the h and dz rows read and written (0.46 GB at 16 x 40,962
 // rows, about 90 µs of HBM time) and the gathers' dependent loads.  Measured at
-// that size, loss and gradient of the error loss: 289 µs, against 2,020 µs with
+// that size, loss and gradient of the error loss: 271 µs, against 2,020 µs with
 // one kernel per operation (dg in FP32, two launches per reduction), the
 // gradient as far from its value in 64 bits as before (4.1e-3 of its norm).
 
@@ -1350,7 +1360,7 @@ __global__ void __launch_bounds__(TB) k_prolong_hp(int n, int nc, int width, con
   double sq = 0.0;
   if (v < n) {
     size_t o = static_cast<size_t>(b) * n + v;
-    float eh = eps[o] - dec_ell::row<0, float, float>(n, width, v, col, val, crs + static_cast<size_t>(b) * nc);
+    float eh = eps[o] - row_of(n, width, v, col, val, crs + static_cast<size_t>(b) * nc);
     eps[o] = eh;
     sq = static_cast<double>(eh) * eh;
   }
@@ -1413,9 +1423,9 @@ __global__ void __launch_bounds__(TB) k_head_back(int n, int B, int nc, int aw, 
     int v = t * 64 + lane, vv = min(v, n - 1);
     float a;
     if constexpr (ERR)
-      a = scale * (g[o + vv] - dec_ell::row<0, float, float>(n, aw, vv, acol, aval, crs + static_cast<size_t>(b) * nc));
+      a = scale * (g[o + vv] - row_of(n, aw, vv, acol, aval, crs + static_cast<size_t>(b) * nc));
     else
-      a = dec_ell::row<0, float, float>(n, aw, vv, acol, aval, g + o);
+      a = row_of(n, aw, vv, acol, aval, g + o);
     float dy = v < n ? -a / D[vv] : 0.0f;
     sums[8] += dy;
     sums[9] += dy * x[o + vv];
@@ -2243,7 +2253,7 @@ void dense(int R, const AT *h, const AT *m, const float *W, const float *b, AT *
 void scale(dec_nn_s &nn, int n, int B, const float *r, hipStream_t st) {
   if (nn.s.n < static_cast<size_t>(B)) nn.s.alloc(B);
   if (nn.spart.n < static_cast<size_t>(B) * kScaleBlocks) nn.spart.alloc(static_cast<size_t>(B) * kScaleBlocks);
-  hipLaunchKernelGGL(k_scale_partial, dim3(kScaleBlocks, B), dim3(TB), 0, st, n, r, nn.spart.p);
+  scale_partial(n, B, r, nn.spart.p, st);
   hipLaunchKernelGGL(k_scale_final, dim3(dec::nblocks(B, 64)), dim3(64), 0, st, n, B, nn.spart.p, nn.s.p);
 }
 
@@ -2446,7 +2456,7 @@ void nn_smooth(dec_nn_s &nn, int lvl, const float *r, float *u, hipStream_t s, b
   // the scale's partial sums (over r in the caller's order); the next kernel
   // adds them (a last-workgroup ticket would need a device-scope fence per
   // workgroup, which writes back the XCD's L2)
-  hipLaunchKernelGGL(k_scale_partial, dim3(kScaleBlocks, 1), dim3(TB), 0, s, n, r, nn.spart.p);
+  scale_partial(n, 1, r, nn.spart.p, s);
   if (n > kInfSmallRows && NL.pi.width >= 1 && NL.pi.width <= 8) {
     // Large levels run over the multigrid level's own numbering, whose BFS
     // blocks keep a row's neighbours close together (the vertex order of a
