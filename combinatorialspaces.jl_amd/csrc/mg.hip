@@ -3154,15 +3154,29 @@ struct Hook {
   Hook &operator=(const Hook &) = delete;
 };
 
+// r = b - A u on the finest level with the per-workgroup sums of r² (rpart),
+// before a cycle of the variant: the mixed variant's cycle takes the residual
+// rounded to float32 in F.f.b and forms none itself, so it is written here.
+// r: where the float64 residual is wanted too, or null.
+void finest_residual(dec_mg_s &mg, int variant, const double *b, const double *u, double *r, hipStream_t s) {
+  Level &F = *mg.lv[0];
+  int nb = dec::nblocks(F.n, kBlock);
+  if (mg.rpart.n < static_cast<size_t>(nb)) fail(DEC_ERR_ARG, "multigrid: residual partials");
+  float *rounded = variant == DEC_SOLVE_MIXED_IR ? F.f.b.p : nullptr;
+  DEC_ELL_WIDTH_SWITCH(F.width, hipLaunchKernelGGL((k_residual_norm<W>), dim3(nb), dim3(kBlock), 0, s, F.n, F.width,
+                                                   F.vcol.p, F.d.vval.p, static_cast<const int *>(nullptr), b, u, r,
+                                                   rounded, mg.rpart.p));
+}
+
+// One cycle; for the mixed variant finest_residual has formed the residual of u.
 void cycle_body(dec_mg_s &mg, int variant, double *u, const double *b, hipStream_t s) {
   Level &F = *mg.lv[0];
   int n = F.n;
   if (variant == DEC_SOLVE_PLAIN_F64) {
     mu_cycle<double>(mg, 0, u, b, 1, false, s);
   } else {
-    // float32 V-cycle on the float64 residual (rounded by the launch that formed
-    // it), correction added in float64: by the cycle's last sweep where it is a
-    // panel sweep, which saves a launch (2.3 µs at 100,000 rows)
+    // float32 V-cycle on the rounded residual (F.f.b), correction added in
+    // float64: by the cycle's last sweep where it is a panel sweep, which saves a launch (2.3 µs at 100,000 rows)
     bool swept = zero_unread<float>(mg, F);
     if (!swept) hipLaunchKernelGGL(k_zero<float>, G(n), dim3(kBlock), 0, s, n, F.f.u.p);
     {
@@ -3273,15 +3287,10 @@ void solve(dec_mg_s &mg, int variant, double tol, int max_cycles, double *u_call
   // refines) and, when `check`, its norm on its way to the host
   auto post = [&](int k, bool check) {
     if (plain && !check) return;
-    int nb = dec::nblocks(n, kBlock);
-    if (mg.rpart.n < static_cast<size_t>(nb)) fail(DEC_ERR_ARG, "multigrid: residual partials");
-    DEC_ELL_WIDTH_SWITCH(F.width, hipLaunchKernelGGL((k_residual_norm<W>), dim3(nb), dim3(kBlock), 0, s, n, F.width,
-                                                     F.vcol.p, F.d.vval.p, static_cast<const int *>(nullptr), b, u,
-                                                     static_cast<double *>(nullptr), plain ? nullptr : F.f.b.p,
-                                                     mg.rpart.p));
+    finest_residual(mg, variant, b, u, nullptr, s);
     if (!check) return;
     double *slot = mg.scal.p + (k % kNormSlots);
-    hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(kBlock), 0, s, nb, mg.rpart.p, slot);
+    hipLaunchKernelGGL(k_sum_rows, dim3(1), dim3(kBlock), 0, s, dec::nblocks(n, kBlock), mg.rpart.p, slot);
     gcheck(hipMemcpyAsync(mg.hnorm + (k % kNormSlots), slot, sizeof(double), hipMemcpyDeviceToHost, s),
            "hipMemcpyAsync");
     gcheck(hipEventRecord(mg.nev[k % kNormSlots], s), "hipEventRecord");
@@ -3439,7 +3448,6 @@ void pcg_solve(dec_mg_s &mg, bool mixed, double tol, int max_iters, double *u_ca
   double *x = io.u;
   const double *b = io.b;
   mg.learned_active = false;
-  if (mg.rpart.n < static_cast<size_t>(nb)) fail(DEC_ERR_ARG, "multigrid: residual partials");
   // a norm on its way to the host: the partial sums part[0..np) added into
   // ring slot k with an event
   auto send = [&](int k, const double *part, int np) {
@@ -3453,11 +3461,10 @@ void pcg_solve(dec_mg_s &mg, bool mixed, double tol, int max_iters, double *u_ca
     gcheck(hipEventSynchronize(mg.nev[k % kNormSlots]), "hipEventSynchronize");
     return std::sqrt(mg.hnorm[k % kNormSlots]) / bn;
   };
-  // the true residual b - A x into F.d.r, its norm to slot k
+  // the true residual b - A x into F.d.r and where the fallback's cycle reads it, its norm to slot k
+  const int fallback = mixed ? DEC_SOLVE_MIXED_IR : DEC_SOLVE_PLAIN_F64;
   auto true_residual = [&](int k) {
-    DEC_ELL_WIDTH_SWITCH(F.width, hipLaunchKernelGGL((k_residual_norm<W>), dim3(nb), dim3(kBlock), 0, s, n, F.width,
-                                                     F.vcol.p, F.d.vval.p, static_cast<const int *>(nullptr), b, x,
-                                                     F.d.r.p, static_cast<float *>(nullptr), mg.rpart.p));
+    finest_residual(mg, fallback, b, x, F.d.r.p, s);
     send(k, mg.rpart.p, nb);
   };
   // CG from the true residual in F.d.r
@@ -3541,9 +3548,8 @@ void pcg_solve(dec_mg_s &mg, bool mixed, double tol, int max_iters, double *u_ca
     c = enq;
     true_residual(c);
     rr = read_norm(c);
-    int variant = mixed ? DEC_SOLVE_MIXED_IR : DEC_SOLVE_PLAIN_F64;
     while (stalled && rr > tol && c < max_iters) {
-      run_cycle(mg, variant, x, b, s);
+      run_cycle(mg, fallback, x, b, s);
       c++;
       true_residual(c);
       rr = read_norm(c);
