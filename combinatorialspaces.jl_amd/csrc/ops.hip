@@ -372,7 +372,8 @@ __device__ __forceinline__ void b_wedge_dd(int blk, int ne, int vec, const int *
     ldt(wa, e, 2, x);
     ldt(wb, e, 2, y);
     ldt(g, e, vec, gg);
-    // every gather is issued; a missing coface reads entry 0 and adds nothing
+    // every gather is issued; a missing coface reads entry 0 (f has one, see
+    // vec_of) and adds nothing
 #pragma unroll
     for (int k = 0; k < N; k++) {
       fa[k] = f[p[k] < 0 ? 0 : p[k]];
@@ -1634,9 +1635,12 @@ void ginv_apply(dec_op_s &op, const T *bvec, T *x, hipStream_t s) {
 template <class T>
 void comp_apply(dec_op_s &op, const T *x, const T *y, T *out, hipStream_t s);
 
-// How the caller's forms may be loaded (see kPer).
+// How the caller's forms may be loaded (see kPer).  The dual-dual wedge's vector
+// path reads entry 0 of the gathered 0-form for a missing coface: on a complex
+// without triangles that form is empty, and every edge goes element by element.
 template <class T>
-int vec_of(const void *x, const void *y, const void *out) {
+int vec_of(const dec_op_s &op, const void *x, const void *y, const void *out) {
+  if (op.impl == I_WDD && (op.m == 0 ? op.cols : op.cols2) == 0) return 0;
   uintptr_t a = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y);
   if (a % 16 == 0) return 2;
   return sizeof(T) == 4 && a % 8 == 0 ? 1 : 0;
@@ -1651,7 +1655,7 @@ void apply_t(dec_op_s &op, const void *xv, const void *yv, void *outv, hipStream
   if (rows == 0) return;
   dim3 g(dec::xcd_grid(rows)), b(256);
   dim3 g2(dec::xcd_grid((static_cast<long long>(rows) + kPer<T> - 1) / kPer<T>));
-  int vec = vec_of<T>(x, y, out);
+  int vec = vec_of<T>(op, x, y, out);
   auto C = [](DBuf<unsigned char> &c) { return reinterpret_cast<const T *>(c.p); };
   // grid of a gather kernel: one workgroup per schedule entry when it has one
   auto gs = [&](dim3 dflt) { return op.sched.p ? dim3(op.nsched) : dflt; };
@@ -1928,7 +1932,7 @@ void apply_group_t(int count, dec_op_s *const *ops, const void *const *xs, const
       GroupOp &o = g.op[k];
       o.impl = op.impl;
       o.rows = static_cast<int>(op.rows);
-      o.vec = vec_of<T>(x, y, outs[q]);
+      o.vec = vec_of<T>(op, x, y, outs[q]);
       o.swap_wdd = op.impl == I_WDD && op.m != 0;
       o.i0 = op.i0.p;
       o.i1 = op.i1.p;
