@@ -2175,8 +2175,6 @@ struct dec_nn_s {
   DBuf<unsigned char> h1, hm1, h2, hm2, h3, dz;  // activation storage (bf16 or f32)
   DBuf<float2> dm;                                 // (dy, signs of h3) per row
   DBuf<int32_t> idx;
-  size_t cap_rows = 0;
-  int cap_mode = -1;
 };
 
 namespace {
@@ -2192,25 +2190,33 @@ Mode mode_of(const dec::NnLevel &L) {
   return narrow(L.p) && narrow(L.pt) ? kTiles : kGeneral;
 }
 
-void ensure(dec_nn_s &nn, size_t rows, Mode mode) {
-  if (rows <= nn.cap_rows && mode == nn.cap_mode) return;
-  size_t as = mode == kPrecise ? 4 : 2;
-  for (auto *b : {&nn.x, &nn.px, &nn.y, &nn.drho, &nn.eps, &nn.crs}) b->alloc(rows);
-  size_t parts = (rows + 255) / 256 + 64;
-  nn.dpart.alloc(parts + 64);
-  for (auto *b : {&nn.h1, &nn.h2, &nn.h3, &nn.dz}) b->alloc(rows * H * as);
+template <class T>
+void grow(DBuf<T> &b, size_t count) {
+  if (b.n < count) b.alloc(count);
+}
+
+// The work buffers of a batch of B samples on level L, each grown to what the
+// launches below write.  The partial sums go by workgroups, which are counted per
+// sample: on a level of fewer rows than a workgroup takes, there is one for each
+// sample however few its rows.
+void ensure(dec_nn_s &nn, const dec::NnLevel &L, int B, Mode mode) {
+  const size_t n = L.n, rows = n * B, as = mode == kPrecise ? 4 : 2;
+  auto groups = [&](size_t per) { return (n + per - 1) / per * B; };  // workgroups of `per` rows over all samples
+  for (auto *b : {&nn.x, &nn.px, &nn.y, &nn.drho, &nn.eps}) grow(*b, rows);
+  grow(nn.crs, static_cast<size_t>(L.nc) * B);
+  grow(nn.dpart, groups(TB));
+  for (auto *b : {&nn.h1, &nn.h2, &nn.h3, &nn.dz}) grow(*b, rows * H * as);
   if (mode == kTiles) {
-    nn.dm.alloc(rows);
-    nn.part.alloc(static_cast<size_t>(kBackBlocks) * NP);
-  } else {
-    nn.c.alloc(rows);
-    nn.tmp.alloc(rows);
-    nn.dg.alloc(rows * 2 * H);
-    for (auto *b : {&nn.hm1, &nn.hm2}) b->alloc(rows * H * as);
-    nn.part.alloc(parts * 2 * H * H);
+    grow(nn.dm, rows);
+    grow(nn.part, static_cast<size_t>(kBackBlocks) * NP);
+    return;
   }
-  nn.cap_rows = rows;
-  nn.cap_mode = mode;
+  for (auto *b : {&nn.c, &nn.tmp}) grow(*b, rows);
+  grow(nn.dg, rows * 2 * H);
+  for (auto *b : {&nn.hm1, &nn.hm2}) grow(*b, rows * H * as);
+  size_t waves = (rows + 255) / 256 + 3;  // (the weights' launch has whole workgroups of four wavefronts)
+  for (size_t need : {groups(TB) * (2 * H + 2), waves * 2 * H * H, groups(TB / H) * H, groups(TB / H) * 2 * H})
+    grow(nn.part, need);
 }
 
 // out[j] = scale · Σ_p part[p·stride + off + j], j < width (kernels above)
@@ -2283,7 +2289,7 @@ void forward_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, c
 void loss_grad_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, const float *e, double *loss_out,
                      hipStream_t st) {
   int n = L.n;
-  ensure(nn, static_cast<size_t>(n) * B, kTiles);
+  ensure(nn, L, B, kTiles);
   scale(nn, n, B, r, st);
   Acts<unsigned short> A = acts<unsigned short>(nn);
   const float *th = nn.th.p;
@@ -2326,7 +2332,7 @@ void forward_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, float
   int n = L.n;
   size_t rows = static_cast<size_t>(n) * B;
   Mode mode = mode_of<AT>(L);
-  ensure(nn, rows, mode);
+  ensure(nn, L, B, mode);
   Acts<AT> A = acts<AT>(nn);
   const float *th = nn.th.p;
   scale(nn, n, B, r, st);
