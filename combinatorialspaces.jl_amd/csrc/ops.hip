@@ -698,12 +698,13 @@ __device__ __forceinline__ void fc_block(double &a, double &b, double *lds) {
   b = ((lds[4] + lds[5]) + lds[6]) + lds[7];
 }
 
-// (Σ part[0..blocks), Σ part[kFcBlocks..kFcBlocks + blocks)) over the launch's
-// blocks, which all launches of a solve share; the same in every block
-__device__ __forceinline__ void fc_sum(const double *__restrict__ part, double &s1, double &s2, double *lds) {
+// (Σ part[0..blocks), Σ part[kFcBlocks..kFcBlocks + blocks)) over the blocks that
+// wrote them, which all launches over the rows share; the same in every block
+__device__ __forceinline__ void fc_sum(const double *__restrict__ part, double &s1, double &s2, double *lds,
+                                       int blocks = gridDim.x) {
   s1 = s2 = 0.0;
 #pragma unroll 4
-  for (int j = threadIdx.x; j < static_cast<int>(gridDim.x); j += 256) {
+  for (int j = threadIdx.x; j < blocks; j += 256) {
     s1 += part[j];
     s2 += part[kFcBlocks + j];
   }
@@ -817,33 +818,47 @@ __global__ __launch_bounds__(256) void k_fcg_first_update(int n, const T *b, con
   fc_partial(a1, a2, partB, lds + 16);
 }
 
-// The stop flag to the host's pinned word, with the even number of the wait
-// that it answers.  (One thread of the launch that tests last.)  The host reads
-// nothing else that the stream wrote, so the store orders nothing.
+// The stopping test of iteration `it` by itself, of the sums that `blocks` blocks
+// left (second sums: r·r; CG: first r·z, BiCGSTAB: ρ), and the stop flag to the
+// host's pinned word with the even number of the wait that it answers.  One
+// workgroup, whose word is the last thing that the solve does: the host starts
+// whatever comes next when it reads the word, on whatever stream, so everything
+// that this launch read has arrived by then (the sums' barrier) and what it
+// wrote is visible (the release).
 struct Tell {
-  unsigned *word = nullptr;
+  unsigned *word = nullptr;  // null: nobody waits (the stream is captured)
   unsigned ticket = 0;
 };
-__device__ __forceinline__ void tell_host(Tell t, bool done) {
-  if (t.word && blockIdx.x == 0 && threadIdx.x == 0)
-    __hip_atomic_store(t.word, t.ticket | (done ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+__global__ __launch_bounds__(256) void k_fc_test(const double *__restrict__ part, int blocks, double *sc, int it,
+                                                 int bicg, double rtol, Tell tell) {
+  __shared__ double lds[32];
+  bool stop = block_stopped(sc);
+  if (!stop) {
+    double rz, rr;
+    fc_sum(part, rz, rr, lds, blocks);
+    stop = rr <= rtol * rtol * sc[CS_BB] || (bicg && rz == 0.0);
+    if (threadIdx.x == 0) {
+      sc[CS_RR] = rr;
+      sc[CS_ITER] = it;
+      sc[CS_RZ0 + (it & 1)] = rz;
+      if (stop) sc[CS_DONE] = 1.0;
+    }
+  }
+  if (tell.word && threadIdx.x == 0)
+    __hip_atomic_store(tell.word, tell.ticket | (stop ? 1u : 0u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Iteration `it` > 0: the stopping test on the residual after `it` updates, then
-// p_new = z + β p_old, q = A p_new and partials p_new·q.  `last` only tests (and
-// tells the host).
+// p_new = z + β p_old, q = A p_new and partials p_new·q.
 template <int W, class T>
 __global__ __launch_bounds__(256) void k_fcg_spmv(int n, int width, const int *__restrict__ col,
                                                   const T *__restrict__ val, const T *__restrict__ z,
                                                   const T *__restrict__ pold, T *__restrict__ pnew,
                                                   T *__restrict__ q, const double *__restrict__ partB,
                                                   double *__restrict__ partA, double *__restrict__ sc, int it,
-                                                  int last, double rtol, Tell tell) {
+                                                  double rtol) {
   __shared__ double lds[32];
-  if (block_stopped(sc)) {
-    if (last) tell_host(tell, true);
-    return;
-  }
+  if (block_stopped(sc)) return;
   // The thread's first row is loaded before the scalars, which it does not need,
   // and every gather is issued at once (14 to 11 µs at 339,000 edges, float64).
   const int i0 = blockIdx.x * 256 + threadIdx.x;
@@ -851,7 +866,7 @@ __global__ __launch_bounds__(256) void k_fcg_spmv(int n, int width, const int *_
   int c0[WP];
   T v0[WP], z0[WP], p0[WP], zi0 = static_cast<T>(0), pi0 = static_cast<T>(0);
   if constexpr (W > 0) {
-    if (!last && i0 < n) {
+    if (i0 < n) {
 #pragma unroll
       for (int k = 0; k < W; k++) {
         size_t o = static_cast<size_t>(k) * n + i0;
@@ -877,8 +892,7 @@ __global__ __launch_bounds__(256) void k_fcg_spmv(int n, int width, const int *_
     sc[CS_RZ0 + (it & 1)] = rz;
     if (conv) sc[CS_DONE] = 1.0;
   }
-  if (last) tell_host(tell, conv);
-  if (conv || last) return;
+  if (conv) return;
   double rzp = sc[CS_RZ0 + ((it - 1) & 1)];
   T beta = static_cast<T>(rzp != 0.0 ? rz / rzp : 0.0);
   double acc = 0.0;
@@ -999,12 +1013,9 @@ template <class T>
 __global__ __launch_bounds__(256) void k_fbi_dir(int n, const T *__restrict__ r, const T *__restrict__ v,
                                                  const T *__restrict__ dinv, T *__restrict__ p, T *__restrict__ y,
                                                  const double *__restrict__ partR, double *__restrict__ sc, int it,
-                                                 int last, double rtol, Tell tell) {
+                                                 double rtol) {
   __shared__ double lds[32];
-  if (block_stopped(sc)) {
-    if (last) tell_host(tell, true);
-    return;
-  }
+  if (block_stopped(sc)) return;
   double rho, rr;
   fc_sum(partR, rho, rr, lds);
   double bb = it == 0 ? rr : sc[CS_BB];
@@ -1016,8 +1027,7 @@ __global__ __launch_bounds__(256) void k_fbi_dir(int n, const T *__restrict__ r,
     sc[CS_RZ0 + (it & 1)] = rho;
     if (stop) sc[CS_DONE] = 1.0;
   }
-  if (last) tell_host(tell, stop);
-  if (stop || last) return;
+  if (stop) return;
   T beta = static_cast<T>(0), omega = static_cast<T>(0);
   if (it > 0) {
     double rhop = sc[CS_RZ0 + ((it - 1) & 1)];
@@ -1588,17 +1598,21 @@ void ginv_apply(dec_op_s &op, const T *bvec, T *x, hipStream_t s) {
     DEC_ELL_WIDTH_SWITCH(E->width, hipLaunchKernelGGL((k_fbi_spmv<W, T>), gf, blk, 0, s, n, E->width, E->col.p,
                                                       E->val.p, xin, out, a, with_qq, part, sc));
   };
-  auto test = [&](int last) {
-    // (no host waits while the stream is captured)
-    Tell word;
-    if (last && cap == hipStreamCaptureStatusNone) word = {op.word.p, op.word.ticket += 2};
+  auto direction = [&]() {
     if (!bicg) {
       DEC_ELL_WIDTH_SWITCH(E->width, hipLaunchKernelGGL((k_fcg_spmv<W, T>), gf, blk, 0, s, n, E->width, E->col.p,
                                                         E->val.p, z, pbuf[it & 1], pbuf[(it + 1) & 1], q, partB,
-                                                        partA, sc, it, last, op.rtol, word));
+                                                        partA, sc, it, op.rtol));
     } else {
-      hipLaunchKernelGGL(k_fbi_dir<T>, gf, blk, 0, s, n, r, q, dinv, p, z, partA, sc, it, last, op.rtol, word);
+      hipLaunchKernelGGL(k_fbi_dir<T>, gf, blk, 0, s, n, r, q, dinv, p, z, partA, sc, it, op.rtol);
     }
+  };
+  auto test = [&]() {
+    // (no host waits while the stream is captured)
+    Tell word;
+    if (cap == hipStreamCaptureStatusNone) word = {op.word.p, op.word.ticket += 2};
+    hipLaunchKernelGGL(k_fc_test, dim3(1), blk, 0, s, bicg ? partA : partB, static_cast<int>(gf.x), sc, it,
+                       bicg ? 1 : 0, op.rtol, word);
   };
   auto iteration = [&]() {
     if (!bicg && it == 0) {
@@ -1607,11 +1621,11 @@ void ginv_apply(dec_op_s &op, const T *bvec, T *x, hipStream_t s) {
       hipLaunchKernelGGL(k_fcg_first_update<T>, gf, blk, 0, s, n, bvec, pbuf[1], q, dinv, x, r, z, partA, partC, partB,
                          sc, op.rtol);
     } else if (!bicg) {
-      test(0);
+      direction();
       hipLaunchKernelGGL(k_fcg_update<T>, gf, blk, 0, s, n, pbuf[(it + 1) & 1], q, dinv, x, r, z, partA, partB, sc,
                          it);
     } else {
-      test(0);                                          // ρ, β, p, y
+      direction();                                      // ρ, β, p, y
       spmv(z, q, rh, 0, partB);                         // v = A y, r̂·v
       hipLaunchKernelGGL(k_fbi_half<T>, gf, blk, 0, s, n, z, q, dinv, x, r, partB, sc, it);
       spmv(z, t, r, 1, partC);                          // t = A z, t·s, t·t
@@ -1625,7 +1639,7 @@ void ginv_apply(dec_op_s &op, const T *bvec, T *x, hipStream_t s) {
   for (int done_it = 0; done_it < op.max_iter; done_it += chunk, chunk = std::min(2 * chunk, kCgChunk)) {
     for (int k = 0; k < chunk && done_it + k < op.max_iter; k++) iteration();
     // test the latest residual now, so that the flag read below sees it
-    if (done_it + chunk >= op.max_iter || cap == hipStreamCaptureStatusNone) test(1);
+    if (done_it + chunk >= op.max_iter || cap == hipStreamCaptureStatusNone) test();
     if (cap != hipStreamCaptureStatusNone) break;
     dec::check_launch("geometric ⋆1⁻¹");
     if (wait_word(op.word, s)) break;

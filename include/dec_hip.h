@@ -173,12 +173,15 @@ int dec_mesh3_export_dual(dec_mesh m, double *dual_point, double *length, double
  *     Geometric ⋆1⁻¹ (FastDEC.jl:744-748, CUDA ext :93-96) is a solve: apply
  *     returns (-⋆1)⁻¹ x from a Jacobi-scaled Krylov iteration on the device
  *     (CG where ⋆1 is symmetric, BiCGSTAB otherwise) stopped at
- *     ‖x - ⋆1 z‖ ≤ 1e-14 ‖x‖ (float64; 1e-6 in float32).  Apply synchronises
- *     the stream to read the stop flag after 2, 6, 14 and then every 8
- *     iterations, except while the stream is captured into a graph (then the
- *     whole budget of 200 (float64) or 100 (float32) iterations is recorded;
- *     those past convergence return at once).  The operator owns work
- *     vectors: one apply at a time.
+ *     ‖x - ⋆1 z‖ ≤ 1e-14 ‖x‖ (float64; 1e-6 in float32).  Apply waits on the
+ *     host for the stop flag after 2, 6, 14 and then every 8 iterations, except
+ *     while the stream is captured into a graph (then the whole budget of 200
+ *     (float64) or 100 (float32) iterations is recorded; those past convergence
+ *     return at once).  out is ready in the stream's order, as for any
+ *     operator.  The operator owns work vectors: one apply at a time; they are
+ *     free when an apply that was not captured returns, so the next one may
+ *     take another stream.  (The composites that hold such a solve go on after
+ *     it with work vectors of their own: order their applies.)
  *  DEC_OP_LAPLACIAN0 (hodge selects ⋆1): fast_laplace_beltrami
  *     (test/Multigrid.jl:46-48) = ∇²(0, sd) form (DiscreteExteriorCalculus.jl:1887-1890).
  *  DEC_OP_AVG01: avg₀₁_mat (FastDEC.jl:874-892).
