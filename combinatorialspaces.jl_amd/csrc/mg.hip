@@ -653,6 +653,11 @@ struct CgState {
 
 constexpr int kCgBlocksMax = 1024;  // partial sums per reduction
 
+// r·r - 2 α r·Ap + α² Ap·Ap is good to about 1e-16 r·r.  Where it is less than
+// this share of r·r, few digits of the next r·r are left, or none: it is then
+// summed from r - α Ap (both forms of the smoother).
+constexpr double kCgCancelled = 1e-6;
+
 inline int cg_blocks(int n) { return std::min(kCgBlocksMax, dec::nblocks(n, kBlock)); }
 
 // Σ part[0..np) in a fixed order, the same in every workgroup: thread t adds
@@ -878,7 +883,18 @@ __global__ void __launch_bounds__(kBlock)
     }
     a = t[3] / t[0];
     double gn = t[3] - 2.0 * a * t[2] + a * a * t[1];
-    gn = gn > 0.0 ? gn : 0.0;
+    if (!(gn > kCgCancelled * t[3])) {
+      // too much cancelled: the sum itself, by every workgroup in the same order (a
+      // pass over r and Ap by each, on the rare step that cuts ‖r‖ a thousandfold)
+      double g[1] = {0.0};
+#pragma unroll 4
+      for (int i = threadIdx.x; i < n; i += kBlock) {
+        double v = next_r(r0[i], a, q0[i]);
+        g[0] = g[0] + v * v;
+      }
+      group_sums<1, kCgWaves, 4>(g, red, half);
+      gn = g[0];
+    }
     double rn = sqrt(gn);
     if (rn <= es || rn + 1.0 <= 1.0) {  // solved: the step still counts
       for (int i = i0; i < n; i += stride) {
@@ -1193,7 +1209,7 @@ __device__ __forceinline__ void cg_run(const CgRows<R> &o, int n, int steps, dou
       }
     }
     if (it + 1 == steps) return;
-    if (!(gn > 1e-6 * gamma)) {
+    if (!(gn > kCgCancelled * gamma)) {
       // too much cancelled: the sum itself (the same branch in every thread)
       g[0] = 0.0;
 #pragma unroll
