@@ -35,9 +35,10 @@ __device__ __forceinline__ float mul<int8_t, float>(int8_t v, float x) {
   return v > 0 ? x : -x;
 }
 
-template <int W, class T, class V>
+// (x of a type X of its own: each product and the sum are in T)
+template <int W, class T, class V, class X>
 __device__ __forceinline__ T row(int n, int width, int r, const int *__restrict__ col, const V *__restrict__ val,
-                                 const T *__restrict__ x) {
+                                 const X *__restrict__ x) {
   T acc = static_cast<T>(0);
   if constexpr (W > 0) {
     int c[W];
@@ -50,7 +51,7 @@ __device__ __forceinline__ T row(int n, int width, int r, const int *__restrict_
       v[k] = val[q];
     }
 #pragma unroll
-    for (int k = 0; k < W; k++) xv[k] = x[c[k] < 0 ? 0 : c[k]];
+    for (int k = 0; k < W; k++) xv[k] = static_cast<T>(x[c[k] < 0 ? 0 : c[k]]);
 #pragma unroll
     for (int k = 0; k < W; k++)
       if (c[k] >= 0) acc = acc + mul<V, T>(v[k], xv[k]);
@@ -69,7 +70,7 @@ __device__ __forceinline__ T row(int n, int width, int r, const int *__restrict_
       }
       if (c[0] < 0) return acc;
 #pragma unroll
-      for (int j = 0; j < 4; j++) xv[j] = x[c[j] < 0 ? 0 : c[j]];
+      for (int j = 0; j < 4; j++) xv[j] = static_cast<T>(x[c[j] < 0 ? 0 : c[j]]);
 #pragma unroll
       for (int j = 0; j < 4; j++)
         if (c[j] >= 0) acc = acc + mul<V, T>(v[j], xv[j]);
@@ -78,7 +79,7 @@ __device__ __forceinline__ T row(int n, int width, int r, const int *__restrict_
       size_t q = static_cast<size_t>(k) * n + r;
       int c = col[q];
       if (c < 0) break;
-      acc = acc + mul<V, T>(val[q], x[c]);
+      acc = acc + mul<V, T>(val[q], static_cast<T>(x[c]));
     }
   }
   return acc;

@@ -1127,18 +1127,28 @@ __global__ void k_pm(int n, T sa, const T *__restrict__ a, T sb, const T *__rest
 
 // out = sa (A xa) + sb (B xb) over two slot-major ELLs of the same rows, sa, sb =
 // ±1: the last step of ℒ_dd and Δᵈ(1) in one launch, in place of two products
-// that are written, read again and added.  The rows' sums are k_ell's.  Bound
-// by the matrices' bytes.
-template <int WA, class VA, int WB, class T>
+// that are written, read again and added.  The rows' sums are k_ell's, A's in the
+// type of xa.  Bound by the matrices' bytes.
+template <int WA, class VA, int WB, class T, class XA>
 __global__ void __launch_bounds__(256)
-    k_ell_pair(int n, int wa, const int *__restrict__ acol, const VA *__restrict__ aval, const T *__restrict__ xa, T sa,
+    k_ell_pair(int n, int wa, const int *__restrict__ acol, const VA *__restrict__ aval, const XA *__restrict__ xa, T sa,
                int wb, const int *__restrict__ bcol, const T *__restrict__ bval, const T *__restrict__ xb, T sb,
                T *__restrict__ out) {
   int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
-  T a = dec_ell::row_upto<WA, T, VA>(n, wa, r, acol, aval, xa);
+  XA a = dec_ell::row_upto<WA, XA, VA>(n, wa, r, acol, aval, xa);
   T b = dec_ell::row_upto<WB, T, T>(n, wb, r, bcol, bval, xb);
-  stn(out + r, sa * a + sb * b);
+  stn(out + r, static_cast<T>(sa * a + sb * b));
+}
+
+// y = A x with float64 products and sums, for a float32 operator whose steps
+// between are not rounded to float32
+template <int W, class V, class X, class Y>
+__global__ void __launch_bounds__(256)
+    k_ell_sum64(int n, int width, const int *__restrict__ col, const V *__restrict__ val, const X *__restrict__ x,
+                Y *__restrict__ y) {
+  int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < n) y[r] = static_cast<Y>(dec_ell::row<W, double, V>(n, width, r, col, val, x));
 }
 
 // ---- coefficient precomputation (float64) ----
@@ -1788,7 +1798,7 @@ void comp_apply(dec_op_s &op, const T *x, const T *y, T *out, hipStream_t s) {
           apply_t<T>(*i12.sub[2], W12(1), nullptr, W12(2), s);
           const dec::Ell<T> &E = ell(star);
           int n = static_cast<int>(op.rows);
-          hipLaunchKernelGGL((k_ell_pair<4, int8_t, 8, T>), dim3(dec::nblocks(n)), dim3(256), 0, s, n, d.sell.width,
+          hipLaunchKernelGGL((k_ell_pair<4, int8_t, 8, T, T>), dim3(dec::nblocks(n)), dim3(256), 0, s, n, d.sell.width,
                              d.sell.col.p, d.sell.val.p, W(0), static_cast<T>(-1), E.width, E.col.p, E.val.p, W12(2),
                              static_cast<T>(-1), out);
           break;
@@ -1805,17 +1815,31 @@ void comp_apply(dec_op_s &op, const T *x, const T *y, T *out, hipStream_t s) {
       break;
     case C_DL1: {  // x -> M x + N ⋆1⁻¹(x) (FastDEC.jl:845-860), M = S D
       A(0, x, nullptr, W(0));
-      A(3, x, nullptr, W(1));
+      // D x in float64 for either type: rounded to float32 between the factors it
+      // would cost M's precision (see create)
+      double *Dx = reinterpret_cast<double *>(op.tmp[1].p);
+      const dec_op_s &D = *op.sub[3];
+      if constexpr (sizeof(T) == 8) A(3, x, nullptr, Dx);
+      else if (D.rows)
+        DEC_ELL_WIDTH_SWITCH(D.ell64.width, hipLaunchKernelGGL((k_ell_sum64<W, double, T, double>),
+                                                               dim3(dec::nblocks(D.rows)), dim3(256), 0, s,
+                                                               static_cast<int>(D.rows), D.ell64.width, D.ell64.col.p,
+                                                               D.ell64.val.p, x, Dx));
       const dec::Ell<T> &S = ell(*op.sub[1]), &N = ell(*op.sub[2]);
-      if (op.rows > 0 && S.width <= 8 && N.width <= 8) {
-        int n = static_cast<int>(op.rows);
-        hipLaunchKernelGGL((k_ell_pair<8, T, 8, T>), dim3(dec::nblocks(n)), dim3(256), 0, s, n, S.width, S.col.p,
-                           S.val.p, W(1), static_cast<T>(1), N.width, N.col.p, N.val.p, W(0), static_cast<T>(1), out);
+      int n = static_cast<int>(op.rows);
+      if (n > 0 && S.width <= 8 && N.width <= 8) {
+        hipLaunchKernelGGL((k_ell_pair<8, T, 8, T, double>), dim3(dec::nblocks(n)), dim3(256), 0, s, n, S.width,
+                           S.col.p, S.val.p, Dx, static_cast<T>(1), N.width, N.col.p, N.val.p, W(0), static_cast<T>(1),
+                           out);
         break;
       }
-      A(1, W(1), nullptr, W(2));
+      T *w2 = W(2);
+      if constexpr (sizeof(T) == 8) A(1, Dx, nullptr, w2);
+      else if (n > 0)
+        DEC_ELL_WIDTH_SWITCH(S.width, hipLaunchKernelGGL((k_ell_sum64<W, T, double, T>), dim3(dec::nblocks(n)),
+                                                         dim3(256), 0, s, n, S.width, S.col.p, S.val.p, Dx, w2));
       A(2, W(0), nullptr, W(3));
-      pm(op.rows, static_cast<T>(1), W(2), static_cast<T>(1), W(3), out);
+      pm(op.rows, static_cast<T>(1), w2, static_cast<T>(1), W(3), out);
       break;
     }
     default:
@@ -3054,8 +3078,9 @@ dec_op_s *create(dec_mesh_s &m, int kind, int dm, int dn, int hodge, int dtype) 
         // row on an interior edge and D = ⋆0⁻¹ d̃1 of a vertex's degree, a third of
         // the rows.  M itself has 19 slots a row: with it the last launch took 25.5
         // µs at 339,000 edges in float64, and takes 11.5 after 5.0 for D x.  Rounding
-        // error of M x by S (D x) over M's, on seven meshes of 120 to 93,000 edges:
-        // float64 0.75 to 0.82, float32 0.86 to 1.28 (the mean 0.99)
+        // error of M x by S (D x) over M's, on eight meshes of 120 to 93,000 edges:
+        // float64 0.75 to 0.82; float32 0.37 to 0.80 with D and D x in float64 and
+        // S's entries in float32 (0.85 to 1.31 with all of it in float32)
         op->comp = C_DL1;
         op->rows = op->cols = ne;
         op->sub.emplace_back(create(m, DEC_OP_INV_HODGE, 1, 0, DEC_GEOMETRIC_HODGE, dtype));
@@ -3066,9 +3091,9 @@ dec_op_s *create(dec_mesh_s &m, int kind, int dm, int dn, int hodge, int dtype) 
         dec::spgemm(t, csr_of(DEC_OP_DIFFERENTIAL, 1, hodge), N);
         op->sub.emplace_back(ell_op(std::move(S), dtype));
         op->sub.emplace_back(ell_op(std::move(N), dtype));
-        op->sub.emplace_back(ell_op(std::move(D), dtype));
+        op->sub.emplace_back(ell_op(std::move(D), DEC_F64));
         add_tmp(ne);
-        add_tmp(nv);
+        add_tmp(f64 ? nv : 2 * static_cast<int64_t>(nv));  // D x, float64
         add_tmp(ne);
         add_tmp(ne);
       } else {
