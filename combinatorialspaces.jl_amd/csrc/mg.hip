@@ -297,7 +297,8 @@ struct Vec2T<float> {
 // to 7 off-diagonal slots, 16 bits each, and the row's own number and colour), the
 // off-diagonal values slot by slot and the diagonal; its halo (the rows of other
 // blocks that its rows name) is a list of fixed stride, and local indices from B
-// on name halo rows.  So a row costs 72 bytes where a slot-major ELL with 32-bit
+// on name halo rows, the last one (a row's unused slots, of value 0) a zero: whatever
+// a row's own value was, an infinity or NaN among them, it doesn't enter its sum.  So a row costs 72 bytes where a slot-major ELL with 32-bit
 // columns and a row number costs 88, a halo value is loaded once per block, and
 // a full block (the first `nfull`, exactly B rows each) needs no table before its
 // loads: they take two round trips (rows, vectors and halo numbers; the halo's
@@ -327,7 +328,7 @@ __global__ void __launch_bounds__(256)
                   const T *__restrict__ zc, double *__restrict__ dot, double *__restrict__ add) {
   constexpr int S = W - 1;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  T *x = reinterpret_cast<T *>(smem_raw), *bl = x + P.B + P.hs;
+  T *x = reinterpret_cast<T *>(smem_raw), *bl = x + P.B + P.hs + 1;
   const int k = blockIdx.x, t = threadIdx.x, nt = blockDim.x;
   int r0, nr;
   if (k < P.nfull) {
@@ -411,6 +412,7 @@ __global__ void __launch_bounds__(256)
     int i = t + m * nt;
     if (i < P.hs) x[P.B + i] = ZERO ? static_cast<T>(0) : hv[m];
   }
+  if (t == 0) x[P.B + P.hs] = static_cast<T>(0);
   __syncthreads();
   int color[R], row[R];
 #pragma unroll
@@ -435,7 +437,7 @@ __global__ void __launch_bounds__(256)
       T xs[S > 0 ? S : 1], s = static_cast<T>(0);
 #pragma unroll
       for (int q = 0; q < S; q++) xs[q] = x[(w[q >> 1] >> (16 * (q & 1))) & 0xffffu];
-      // (a pad names the row itself with the value 0: it leaves the sum as it is)
+      // (a pad is 0 times the zero: it leaves the sum as it is)
 #pragma unroll
       for (int q = 0; q < S; q++) s = s + off[m][q] * xs[q];
       x[row[m]] = (bv[m] - s) / dg[m];
@@ -497,7 +499,7 @@ __global__ void k_build_panels(int n, int width, int B, int hs, const int *__res
   for (int i = threadIdx.x; i < nr; i += blockDim.x) {
     int r = order[r0 + i], q = 0;
     unsigned int w[8];
-    for (int j = 0; j < 8; j++) w[j] = static_cast<unsigned int>(r - r0);
+    for (int j = 0; j < 8; j++) w[j] = static_cast<unsigned int>(B + hs);
     double d = 0.0;
     double *o = off + static_cast<size_t>(r0) * S + i;
     for (int sl = 0; sl < width; sl++) {
@@ -1675,10 +1677,11 @@ struct Tail {
 constexpr int kTailRows = 3 * kFuseThreads;  // 12-bit numbers, three rows a thread
 constexpr int kTailZ = 16;                   // rows of C in a workgroup
 
-// x (later the chunks' parts of 16 rows of Z r), w, and C's right-hand side
+// x and a zero, which a row's unused slots name (later the chunks' parts of 16 rows
+// of Z r), w, and C's right-hand side
 __host__ __device__ inline int tail_x(int n, int nc) {
   int parts = coarse_chunks(nc) * kTailZ;
-  return n > parts ? n : parts;
+  return n + 1 > parts ? n + 1 : parts;
 }
 inline size_t tail_lds(int n, int nc, size_t bytes) {
   return (static_cast<size_t>(tail_x(n, nc)) + n + nc) * bytes;
@@ -1690,7 +1693,8 @@ __global__ void k_build_tail(const LevelDesc<double> A, int S, uint4 *__restrict
   if (q >= A.n) return;
   unsigned int v = static_cast<unsigned int>(A.rowid[q]), w[8], at = 0, k = 0, c = 0;
   while (static_cast<int>(c) + 1 < A.ncolors && q >= A.cstart[c + 1]) c++;
-  for (int j = 0; j < 8; j++) w[j] = v;
+  for (int j = 0; j < 7; j++) w[j] = static_cast<unsigned int>(A.n);
+  w[7] = v;
   for (int sl = 0; sl < A.width; sl++) {
     size_t o = static_cast<size_t>(sl) * A.n + q;
     int cc = A.col[o];
@@ -1774,6 +1778,7 @@ __global__ void __launch_bounds__(kFuseThreads)
       w[r] = b[r];
     }
   }
+  if (tid == 0) x[n] = static_cast<T>(0);
   __syncthreads();
   o.rhs(w);
   __syncthreads();
@@ -1877,6 +1882,7 @@ __global__ void __launch_bounds__(kFuseThreads)
     if (r < n) w[r] = b[r];
   }
   for (int i = tid; i < nc; i += kFuseThreads) rl[i] = z[i];
+  if (tid == 0) x[n] = static_cast<T>(0);
   o.load(A);
   __syncthreads();
   o.rhs(w);
@@ -2866,7 +2872,7 @@ void panel_sweep(Level &L, const T *b, const T *src, T *dst, bool post, bool zer
               reinterpret_cast<const V2 *>(V.pown_w.p),
               reinterpret_cast<const V2 *>(V.phalo_w.p)};
   int nt = panel_threads(P.B);
-  size_t lds = static_cast<size_t>(2 * P.B + P.hs) * sizeof(T);
+  size_t lds = static_cast<size_t>(2 * P.B + P.hs + 1) * sizeof(T);
   int rev = post ? 1 : 0;
 #define DEC_PANEL(WW, RR, ZZ) \
   hipLaunchKernelGGL((k_panel_sweep<WW, T, RR, ZZ>), dim3(L.nblk), dim3(nt), lds, s, P, b, src, dst, rev, zc, dot, add)
