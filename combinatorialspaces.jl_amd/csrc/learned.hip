@@ -1201,9 +1201,12 @@ __global__ void k_hp_grad(int n, float scale, const float *__restrict__ eh, cons
 // dh = dz W_ownᵀ + q W_nbᵀ (P h and dz Wᵀ are never stored): the only rows that
 // are gathered are dz's own 64 bytes, and at the head 8 bytes (dy, mask) from
 // which a neighbour's dz3 is formed again.  q is summed in FP32 and enters the
-// matrix products as the sum of two BF16 values.  Each workgroup adds its
-// tiles' parameter sums in registers and writes one row of `part`
-// (kBackBlocks rows of NP); k_reduce_params adds the rows in double.
+// matrix products as the sum of two BF16 values.  A wavefront adds the parameter
+// sums of kBackTiles tiles (256 rows) in float32 registers; then they go to sums in
+// double over the workgroup (each wavefront holds a quarter of the parameters), and
+// in the end the workgroup writes one row of `part` (kBackBlocks rows of NP);
+// k_reduce_params adds the rows in double.  So a large batch means no longer
+// float32 sums.
 //
 // What bounds them: the h and dz rows read and written (0.46 GB at 16 x 40,962
 // rows, about 90 µs of HBM time) and the gathers' dependent loads.  Measured at
@@ -1212,6 +1215,7 @@ __global__ void k_hp_grad(int n, float scale, const float *__restrict__ eh, cons
 // gradient as far from its value in 64 bits as before (4.1e-3 of its norm).
 
 constexpr int kBackBlocks = 768;           // at most, three a CU; a multiple of 8
+constexpr int kBackTiles = 4;              // tiles that a wavefront adds in float32
 constexpr int kBackPitch = 4 * H + 8;      // bf16 per LDS row: [dz | q high | q low | h] plus padding
 
 // x = r / s, P x and the layer-1 rows h1 (the values of k_input).
@@ -1373,22 +1377,6 @@ __global__ void __launch_bounds__(TB) k_prolong_hp(int n, int nc, int width, con
   if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = sh[0];
 }
 
-// Σ over the workgroup's four waves of 64 x K per-lane values (K at a time in LDS), lane l of wave 0 holding it
-template <int K>
-__device__ __forceinline__ void add_waves(float (&v)[K], float *lds) {
-  int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < K; k++) lds[(w * K + k) * 64 + lane] = v[k];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < K; k++) {
-    v[k] = 0.0f;
-#pragma unroll
-    for (int q = 0; q < kInfWaves; q++) v[k] = v[k] + lds[(q * K + k) * 64 + lane];
-  }
-}
-
 // The tiles of this wavefront: XCD x (workgroups ≡ x mod 8) takes the x-th
 // contiguous eighth of the `total` tiles, its wavefronts side by side.
 __device__ __forceinline__ void wave_tiles(int total, int &first, int &end, int &step) {
@@ -1408,65 +1396,77 @@ __global__ void __launch_bounds__(TB) k_head_back(int n, int B, int nc, int aw, 
                                                   const float *__restrict__ crs, float scale,
                                                   const float *__restrict__ D, const float *__restrict__ x,
                                                   const unsigned short *__restrict__ h3, float2 *__restrict__ dm,
-                                                  float *__restrict__ part_out) {
-  __shared__ float red[kInfWaves * 10 * 64];
+                                                  float *__restrict__ part_out, int runs) {
+  constexpr int kSums = H + 2;  // Σ dy h3, Σ dy, Σ dy x
+  __shared__ float red[kInfWaves][kSums];
   const int lane = threadIdx.x & 63, sub = lane >> 2, part = lane & 3;
   const int T = (n + 63) / 64;
-  float sums[10];  // Σ dy h3 of the features 8 part .. + 7, then Σ dy and Σ dy x of the lane's rows
-#pragma unroll
-  for (int k = 0; k < 10; k++) sums[k] = 0.0f;
   int w, wend, step;
   wave_tiles(B * T, w, wend, step);
-  for (; w < wend; w += step) {
-    int b = w / T, t = w - b * T;
-    size_t o = static_cast<size_t>(b) * n;
-    int v = t * 64 + lane, vv = min(v, n - 1);
-    float a;
-    if constexpr (ERR)
-      a = scale * (g[o + vv] - row_of(n, aw, vv, acol, aval, crs + static_cast<size_t>(b) * nc));
-    else
-      a = row_of(n, aw, vv, acol, aval, g + o);
-    float dy = v < n ? -a / D[vv] : 0.0f;
-    sums[8] += dy;
-    sums[9] += dy * x[o + vv];
+  double total = 0.0;  // of the parameter threadIdx.x
+#pragma unroll 1
+  for (int run = 0; run < runs; run++) {
+    float sums[10];  // Σ dy h3 of the features 8 part .. + 7, then Σ dy and Σ dy x of the lane's rows
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      int r = t * 64 + 16 * q + sub;
-      uint4 hr = *reinterpret_cast<const uint4 *>(h3 + (o + min(r, n - 1)) * H + 8 * part);
-      float d = __shfl(dy, 16 * q + sub);
-      float f[8];
-      unpack8(hr, f);
-      unsigned int m = 0;
+    for (int k = 0; k < 10; k++) sums[k] = 0.0f;
+#pragma unroll 1
+    for (int j = 0; j < kBackTiles && w < wend; j++, w += step) {
+      int b = w / T, t = w - b * T;
+      size_t o = static_cast<size_t>(b) * n;
+      int v = t * 64 + lane, vv = min(v, n - 1);
+      float a;
+      if constexpr (ERR)
+        a = scale * (g[o + vv] - row_of(n, aw, vv, acol, aval, crs + static_cast<size_t>(b) * nc));
+      else
+        a = row_of(n, aw, vv, acol, aval, g + o);
+      float dy = v < n ? -a / D[vv] : 0.0f;
+      sums[8] += dy;
+      sums[9] += dy * x[o + vv];
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        sums[e] += d * f[e];
-        m |= (f[e] > 0.0f ? 1u : 0u) << e;
+      for (int q = 0; q < 4; q++) {
+        int r = t * 64 + 16 * q + sub;
+        uint4 hr = *reinterpret_cast<const uint4 *>(h3 + (o + min(r, n - 1)) * H + 8 * part);
+        float d = __shfl(dy, 16 * q + sub);
+        float f[8];
+        unpack8(hr, f);
+        unsigned int m = 0;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          sums[e] += d * f[e];
+          m |= (f[e] > 0.0f ? 1u : 0u) << e;
+        }
+        m <<= 8 * part;
+        m |= __shfl_xor(m, 1);
+        m |= __shfl_xor(m, 2);
+        if (part == 0 && r < n) dm[o + r] = make_float2(d, __uint_as_float(m));
       }
-      m <<= 8 * part;
-      m |= __shfl_xor(m, 1);
-      m |= __shfl_xor(m, 2);
-      if (part == 0 && r < n) dm[o + r] = make_float2(d, __uint_as_float(m));
+    }
+#pragma unroll
+    for (int off = 4; off < 64; off <<= 1)
+#pragma unroll
+      for (int k = 0; k < 8; k++) sums[k] += __shfl_xor(sums[k], off);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      sums[8] += __shfl_xor(sums[8], off);
+      sums[9] += __shfl_xor(sums[9], off);
+    }
+    __syncthreads();
+    if (lane < 4) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) red[threadIdx.x >> 6][8 * part + e] = sums[e];
+    }
+    if (lane == 0) {
+      red[threadIdx.x >> 6][H] = sums[8];
+      red[threadIdx.x >> 6][H + 1] = sums[9];
+    }
+    __syncthreads();
+    if (threadIdx.x < kSums) {
+#pragma unroll
+      for (int q = 0; q < kInfWaves; q++) total = total + static_cast<double>(red[q][threadIdx.x]);
     }
   }
-#pragma unroll
-  for (int off = 4; off < 64; off <<= 1)
-#pragma unroll
-    for (int k = 0; k < 8; k++) sums[k] += __shfl_xor(sums[k], off);
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    sums[8] += __shfl_xor(sums[8], off);
-    sums[9] += __shfl_xor(sums[9], off);
-  }
-  add_waves<10>(sums, red);
-  float *out = part_out + static_cast<size_t>(blockIdx.x) * NP;
-  if (threadIdx.x < 4) {
-#pragma unroll
-    for (int e = 0; e < 8; e++) out[OWO + 8 * part + e] = sums[e];
-    if (part == 0) {
-      out[OBO] = sums[8];
-      out[OAL] = sums[9];
-    }
-  }
+  // (wo, bo and alpha follow one another)
+  if (threadIdx.x < kSums) part_out[static_cast<size_t>(blockIdx.x) * NP + OWO + threadIdx.x] = static_cast<float>(total);
 }
 
 // Four consecutive rows' entries of one LDS column, as an MFMA operand over rows:
@@ -1487,11 +1487,11 @@ __global__ void __launch_bounds__(TB, 3)
     k_layer_back(int n, int B, const int *__restrict__ ptcol, const float *__restrict__ ptval,
                  const unsigned short *__restrict__ dzin, const float2 *__restrict__ dm, const float *__restrict__ wo,
                  const unsigned short *__restrict__ hb, const float *__restrict__ Wt, unsigned short *__restrict__ dzout,
-                 const float *__restrict__ x, const float *__restrict__ px, float *__restrict__ part_out, int ow,
-                 int ob_below, int ob_self) {
+                 const float *__restrict__ x, const float *__restrict__ px, float *__restrict__ part_out, int runs,
+                 int ow, int ob_below, int ob_self) {
   __shared__ __align__(16) unsigned short rows_s[kInfWaves][2][16 * kBackPitch];
   __shared__ float2 xs_s[HEAD ? 1 : kInfWaves][64];
-  static_assert(sizeof(rows_s) >= kInfWaves * 32 * 64 * sizeof(float), "the sums at the end");
+  static_assert(sizeof(rows_s) >= kInfWaves * (32 * 64 + 3 * H) * sizeof(float), "the sums of a run");
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4, sub = lane >> 2, part = lane & 3;
   const int T = (n + 63) / 64;
@@ -1512,14 +1512,6 @@ __global__ void __launch_bounds__(TB, 3)
 #pragma unroll
     for (int e = 0; e < 8; e++) wl[e] = wo[8 * part + e];
   }
-  float4_t aO[2][2], aN[2][2];  // dW tiles: features 16 ft.., columns 16 jt..
-#pragma unroll
-  for (int ft = 0; ft < 2; ft++)
-#pragma unroll
-    for (int jt = 0; jt < 2; jt++) aO[ft][jt] = aN[ft][jt] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  float osum[8], bsum[2] = {0.0f, 0.0f}, w1[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int e = 0; e < 8; e++) osum[e] = 0.0f;
   int wt, wend, step;
   wave_tiles(B * T, wt, wend, step);
   // One 16-row group at a time, four to a tile: the rows pass through 8.7 KB of
@@ -1531,140 +1523,157 @@ __global__ void __launch_bounds__(TB, 3)
   // workgroups a CU, 58 and 41; held to four, with spills, 61 and 42.
   int c[W];
   float pv[W];
-  for (; wt < wend; wt += step) {
-    const int b = wt / T, t = wt - b * T;
-    const size_t o = static_cast<size_t>(b) * n;
-    own_slots<W>(n, t * 64 + lane, ptcol, ptval, c, pv);
-    if constexpr (!HEAD) {
-      size_t i = o + min(t * 64 + lane, n - 1);
-      xs_s[wv][lane] = make_float2(x[i], px[i]);
-    }
+  // the sums in double: wave w holds dW's registers k = w, w + 4, ... (see v below), thread t < kCols the t-th of
+  // the columns' sums: the bias below, then dz's own (HEAD) or W1's
+  constexpr int kCols = HEAD ? 2 * H : 3 * H;
+  double dW[32 / kInfWaves] = {}, dcol = 0.0;
 #pragma unroll 1
-    for (int g = 0; g < 4; g++) {
-      unsigned short *rows = rows_s[wv][g & 1];
-      const int r = t * 64 + 16 * g + sub;
-      const size_t rr = o + min(r, n - 1);
-      uint4 hr, own, a[HEAD ? 1 : W];
-      float2 od, nd[HEAD ? W : 1];
-      hr = *reinterpret_cast<const uint4 *>(hb + rr * H + 8 * part);
-      if constexpr (HEAD) od = dm[rr];
-      else own = *reinterpret_cast<const uint4 *>(dzin + rr * H + 8 * part);
-      unsigned int have = 0;  // the row's slots that are not pads
+  for (int run = 0; run < runs; run++) {
+    float4_t aO[2][2], aN[2][2];  // dW tiles: features 16 ft.., columns 16 jt..
 #pragma unroll
-      for (int k = 0; k < W; k++) {
-        int cg = __shfl(c[k], 16 * g + sub);
-        have |= (cg >= 0 ? 1u : 0u) << k;
-        size_t i = o + (cg < 0 ? 0 : cg);
-        if constexpr (HEAD) nd[k] = dm[i];
-        else a[k] = *reinterpret_cast<const uint4 *>(dzin + i * H + 8 * part);
+    for (int ft = 0; ft < 2; ft++)
+#pragma unroll
+      for (int jt = 0; jt < 2; jt++) aO[ft][jt] = aN[ft][jt] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    float osum[8], bsum[2] = {0.0f, 0.0f}, w1[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int e = 0; e < 8; e++) osum[e] = 0.0f;
+#pragma unroll 1
+    for (int tile = 0; tile < kBackTiles && wt < wend; tile++, wt += step) {
+      const int b = wt / T, t = wt - b * T;
+      const size_t o = static_cast<size_t>(b) * n;
+      own_slots<W>(n, t * 64 + lane, ptcol, ptval, c, pv);
+      if constexpr (!HEAD) {
+        size_t i = o + min(t * 64 + lane, n - 1);
+        xs_s[wv][lane] = make_float2(x[i], px[i]);
       }
-      float q[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) q[e] = 0.0f;
-      float vg[W];
-#pragma unroll
-      for (int k = 0; k < W; k++) vg[k] = __shfl(pv[k], 16 * g + sub);
-      uint4 mine;
-      if constexpr (HEAD) {
-        auto form = [&](float2 d, bool keep) {
-          unsigned int m = keep ? __float_as_uint(d.y) >> (8 * part) : 0u;
-          float z[8];
-#pragma unroll
-          for (int e = 0; e < 8; e++) z[e] = (m >> e) & 1u ? d.x * wl[e] : 0.0f;
-          return pack8(z);
-        };
-        mine = form(od, r < n);
-        float f[8];
-        unpack8(mine, f);
-#pragma unroll
-        for (int e = 0; e < 8; e++) osum[e] += f[e];
+#pragma unroll 1
+      for (int g = 0; g < 4; g++) {
+        unsigned short *rows = rows_s[wv][g & 1];
+        const int r = t * 64 + 16 * g + sub;
+        const size_t rr = o + min(r, n - 1);
+        uint4 hr, own, a[HEAD ? 1 : W];
+        float2 od, nd[HEAD ? W : 1];
+        hr = *reinterpret_cast<const uint4 *>(hb + rr * H + 8 * part);
+        if constexpr (HEAD) od = dm[rr];
+        else own = *reinterpret_cast<const uint4 *>(dzin + rr * H + 8 * part);
+        unsigned int have = 0;  // the row's slots that are not pads
 #pragma unroll
         for (int k = 0; k < W; k++) {
-          unpack8(form(nd[k], have >> k & 1u), f);
-#pragma unroll
-          for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
+          int cg = __shfl(c[k], 16 * g + sub);
+          have |= (cg >= 0 ? 1u : 0u) << k;
+          size_t i = o + (cg < 0 ? 0 : cg);
+          if constexpr (HEAD) nd[k] = dm[i];
+          else a[k] = *reinterpret_cast<const uint4 *>(dzin + i * H + 8 * part);
         }
-      } else {
-        mine = keep_if(own, r < n);
+        float q[8];
 #pragma unroll
-        for (int k = 0; k < W; k++) {
+        for (int e = 0; e < 8; e++) q[e] = 0.0f;
+        float vg[W];
+#pragma unroll
+        for (int k = 0; k < W; k++) vg[k] = __shfl(pv[k], 16 * g + sub);
+        uint4 mine;
+        if constexpr (HEAD) {
+          auto form = [&](float2 d, bool keep) {
+            unsigned int m = keep ? __float_as_uint(d.y) >> (8 * part) : 0u;
+            float z[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) z[e] = (m >> e) & 1u ? d.x * wl[e] : 0.0f;
+            return pack8(z);
+          };
+          mine = form(od, r < n);
           float f[8];
-          unpack8(keep_if(a[k], have >> k & 1u), f);
+          unpack8(mine, f);
 #pragma unroll
-          for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
-        }
-      }
-      uint4 hi = pack8(q);
-      float fh[8];
-      unpack8(hi, fh);
+          for (int e = 0; e < 8; e++) osum[e] += f[e];
 #pragma unroll
-      for (int e = 0; e < 8; e++) q[e] = q[e] - fh[e];
-      unsigned short *d = rows + sub * kBackPitch + 8 * part;
-      *reinterpret_cast<uint4 *>(d) = mine;
-      *reinterpret_cast<uint4 *>(d + H) = hi;
-      *reinterpret_cast<uint4 *>(d + 2 * H) = pack8(q);
-      *reinterpret_cast<uint4 *>(d + 3 * H) = keep_if(hr, r < n);
-      wave_sync();
-      // dW += hᵀ dz, hᵀ q
-      unsigned short *base = rows + 4 * lg * kBackPitch;
-      short4_t A[2], Z[2], Q[2], L[2];
+          for (int k = 0; k < W; k++) {
+            unpack8(form(nd[k], have >> k & 1u), f);
 #pragma unroll
-      for (int k = 0; k < 2; k++) {
-        A[k] = lds_col4(base + 3 * H + 16 * k, li);
-        Z[k] = lds_col4(base + 16 * k, li);
-        Q[k] = lds_col4(base + H + 16 * k, li);
-        L[k] = lds_col4(base + 2 * H + 16 * k, li);
-      }
+            for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
+          }
+        } else {
+          mine = keep_if(own, r < n);
 #pragma unroll
-      for (int ft = 0; ft < 2; ft++)
+          for (int k = 0; k < W; k++) {
+            float f[8];
+            unpack8(keep_if(a[k], have >> k & 1u), f);
 #pragma unroll
-        for (int jt = 0; jt < 2; jt++) {
-          aO[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], Z[jt], aO[ft][jt], 0, 0, 0);
-          aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], Q[jt], aN[ft][jt], 0, 0, 0);
-          aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], L[jt], aN[ft][jt], 0, 0, 0);
-        }
-      // dh, masked by the signs of h
-      const unsigned short *rp = rows + li * kBackPitch + 4 * lg;
-      short4_t Zr[2] = {lds4(rp), lds4(rp + 16)}, Qr[2] = {lds4(rp + H), lds4(rp + H + 16)},
-               Lr[2] = {lds4(rp + 2 * H), lds4(rp + 2 * H + 16)};
-      wave_sync();
-#pragma unroll
-      for (int jt = 0; jt < 2; jt++) {
-        float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
-          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Zr[ks], Bo[jt][ks], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Lr[ks], Bn[jt][ks], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Qr[ks], Bn[jt][ks], acc, 0, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          // h is zero in rows past the end, so those add nothing; A holds h of
-          // the accumulator's own rows and column
-          float gv = bf2f(static_cast<unsigned short>(A[jt][i])) > 0.0f ? acc[i] : 0.0f;
-          bsum[jt] += gv;
-          if constexpr (HEAD) {
-            rows[(4 * lg + i) * kBackPitch + 16 * jt + li] = f2bf(gv);
-          } else {
-            float2 xp = xs_s[wv][16 * g + 4 * lg + i];
-            w1[jt] += xp.x * gv;
-            w1[2 + jt] += xp.y * gv;
+            for (int e = 0; e < 8; e++) q[e] = q[e] + vg[k] * f[e];
           }
         }
-      }
-      if constexpr (HEAD) {
+        uint4 hi = pack8(q);
+        float fh[8];
+        unpack8(hi, fh);
+#pragma unroll
+        for (int e = 0; e < 8; e++) q[e] = q[e] - fh[e];
+        unsigned short *d = rows + sub * kBackPitch + 8 * part;
+        *reinterpret_cast<uint4 *>(d) = mine;
+        *reinterpret_cast<uint4 *>(d + H) = hi;
+        *reinterpret_cast<uint4 *>(d + 2 * H) = pack8(q);
+        *reinterpret_cast<uint4 *>(d + 3 * H) = keep_if(hr, r < n);
         wave_sync();
-        if (r < n)
-          *reinterpret_cast<uint4 *>(dzout + (o + r) * H + 8 * part) =
-              *reinterpret_cast<const uint4 *>(rows + sub * kBackPitch + 8 * part);
+        // dW += hᵀ dz, hᵀ q
+        unsigned short *base = rows + 4 * lg * kBackPitch;
+        short4_t A[2], Z[2], Q[2], L[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          A[k] = lds_col4(base + 3 * H + 16 * k, li);
+          Z[k] = lds_col4(base + 16 * k, li);
+          Q[k] = lds_col4(base + H + 16 * k, li);
+          L[k] = lds_col4(base + 2 * H + 16 * k, li);
+        }
+#pragma unroll
+        for (int ft = 0; ft < 2; ft++)
+#pragma unroll
+          for (int jt = 0; jt < 2; jt++) {
+            aO[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], Z[jt], aO[ft][jt], 0, 0, 0);
+            aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], Q[jt], aN[ft][jt], 0, 0, 0);
+            aN[ft][jt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[ft], L[jt], aN[ft][jt], 0, 0, 0);
+          }
+        // dh, masked by the signs of h
+        const unsigned short *rp = rows + li * kBackPitch + 4 * lg;
+        short4_t Zr[2] = {lds4(rp), lds4(rp + 16)}, Qr[2] = {lds4(rp + H), lds4(rp + H + 16)},
+                 Lr[2] = {lds4(rp + 2 * H), lds4(rp + 2 * H + 16)};
+        wave_sync();
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++) {
+          float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int ks = 0; ks < 2; ks++) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Zr[ks], Bo[jt][ks], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Lr[ks], Bn[jt][ks], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(Qr[ks], Bn[jt][ks], acc, 0, 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            // h is zero in rows past the end, so those add nothing; A holds h of
+            // the accumulator's own rows and column
+            float gv = bf2f(static_cast<unsigned short>(A[jt][i])) > 0.0f ? acc[i] : 0.0f;
+            bsum[jt] += gv;
+            if constexpr (HEAD) {
+              rows[(4 * lg + i) * kBackPitch + 16 * jt + li] = f2bf(gv);
+            } else {
+              float2 xp = xs_s[wv][16 * g + 4 * lg + i];
+              w1[jt] += xp.x * gv;
+              w1[2 + jt] += xp.y * gv;
+            }
+          }
+        }
+        if constexpr (HEAD) {
+          wave_sync();
+          if (r < n)
+            *reinterpret_cast<uint4 *>(dzout + (o + r) * H + 8 * part) =
+                *reinterpret_cast<const uint4 *>(rows + sub * kBackPitch + 8 * part);
+        }
       }
     }
-  }
-  // the wavefronts' sums into one row of partials
-  float *out = part_out + static_cast<size_t>(blockIdx.x) * NP;
-  float *lds = reinterpret_cast<float *>(rows_s);
-  {
-    float v[32];
+    // the run's sums into those in double.  (The thread's number as a value the compiler knows nothing about: the
+    // addresses made from it are not kept in registers over the tiles.)
+    unsigned int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const unsigned int l = tid & 63, w = tid >> 6;
+    float *lds = reinterpret_cast<float *>(rows_s), *cols = lds + kInfWaves * 32 * 64;
+    float v[32];  // own rows of W, neighbour rows; each by feature tile, column tile and register
 #pragma unroll
     for (int ft = 0; ft < 2; ft++)
 #pragma unroll
@@ -1674,47 +1683,52 @@ __global__ void __launch_bounds__(TB, 3)
           v[(ft * 2 + jt) * 4 + i] = aO[ft][jt][i];
           v[16 + (ft * 2 + jt) * 4 + i] = aN[ft][jt][i];
         }
-    add_waves<32>(v, lds);
-    if (threadIdx.x < 64) {
+    float c6[HEAD ? 2 : 6];
 #pragma unroll
-      for (int ft = 0; ft < 2; ft++)
-#pragma unroll
-        for (int jt = 0; jt < 2; jt++)
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            int f = 16 * ft + 4 * lg + i, j = 16 * jt + li;
-            out[ow + f * H + j] = v[(ft * 2 + jt) * 4 + i];
-            out[ow + (H + f) * H + j] = v[16 + (ft * 2 + jt) * 4 + i];
-          }
+    for (int k = 0; k < (HEAD ? 2 : 6); k++) {
+      c6[k] = k < 2 ? bsum[k & 1] : w1[(k - 2) & 3];
+      c6[k] += __shfl_xor(c6[k], 16);
+      c6[k] += __shfl_xor(c6[k], 32);
     }
-  }
-  float v[6] = {bsum[0], bsum[1], w1[0], w1[1], w1[2], w1[3]};
+    if constexpr (HEAD) {
 #pragma unroll
-  for (int k = 0; k < 6; k++) {
-    v[k] += __shfl_xor(v[k], 16);
-    v[k] += __shfl_xor(v[k], 32);
-  }
-  add_waves<6>(v, lds);
-  if (threadIdx.x < 16) {
-    out[ob_below + li] = v[0];
-    out[ob_below + 16 + li] = v[1];
-    if constexpr (!HEAD) {
-      out[OW1 + li] = v[2];
-      out[OW1 + 16 + li] = v[3];
-      out[OW1 + H + li] = v[4];
-      out[OW1 + H + 16 + li] = v[5];
+      for (int off = 4; off < 64; off <<= 1)
+#pragma unroll
+        for (int e = 0; e < 8; e++) osum[e] += __shfl_xor(osum[e], off);
     }
-  }
-  if constexpr (HEAD) {
+    __syncthreads();
 #pragma unroll
-    for (int off = 4; off < 64; off <<= 1)
+    for (int k = 0; k < 32; k++) lds[(w * 32 + k) * 64 + l] = v[k];
+    if (l < 16) {
 #pragma unroll
-      for (int e = 0; e < 8; e++) osum[e] += __shfl_xor(osum[e], off);
-    add_waves<8>(osum, lds);
-    if (threadIdx.x < 4) {
-#pragma unroll
-      for (int e = 0; e < 8; e++) out[ob_self + 8 * part + e] = osum[e];
+      for (int k = 0; k < (HEAD ? 2 : 6); k++) cols[w * kCols + 16 * k + l] = c6[k];
     }
+    if constexpr (HEAD) {
+      if (l < 4) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) cols[w * kCols + H + 8 * l + e] = osum[e];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 32 / kInfWaves; j++)
+#pragma unroll
+      for (int q = 0; q < kInfWaves; q++) dW[j] = dW[j] + static_cast<double>(lds[(q * 32 + kInfWaves * j + w) * 64 + l]);
+    if (tid < kCols) {
+#pragma unroll
+      for (int q = 0; q < kInfWaves; q++) dcol = dcol + static_cast<double>(cols[q * kCols + tid]);
+    }
+    __syncthreads();
+  }
+  float *out = part_out + static_cast<size_t>(blockIdx.x) * NP;
+#pragma unroll
+  for (int j = 0; j < 32 / kInfWaves; j++) {
+    int k = kInfWaves * j + wv, f = H * (k >> 4) + 16 * ((k >> 3) & 1) + 4 * lg + (k & 3), col = 16 * ((k >> 2) & 1) + li;
+    out[ow + f * H + col] = static_cast<float>(dW[j]);
+  }
+  if (threadIdx.x < kCols) {
+    int t = threadIdx.x, second = HEAD ? ob_self : OW1;
+    out[t < H ? ob_below + t : second + t - H] = static_cast<float>(dcol);
   }
 }
 
@@ -2208,8 +2222,7 @@ void ensure(dec_nn_s &nn, const dec::NnLevel &L, int B, Mode mode) {
   for (auto *b : {&nn.h1, &nn.h2, &nn.h3, &nn.dz}) grow(*b, rows * H * as);
   if (mode == kTiles) {
     grow(nn.dm, rows);
-    grow(nn.part, static_cast<size_t>(kBackBlocks) * NP);
-    return;
+    return;  // (the partial sums: loss_grad_tiles)
   }
   for (auto *b : {&nn.c, &nn.tmp}) grow(*b, rows);
   grow(nn.dg, rows * 2 * H);
@@ -2269,6 +2282,17 @@ int tile_count(int n, int B) {
   return static_cast<int>(t);
 }
 
+// Workgroups of the backward launches, and how often each hands its sums over: an
+// XCD has at most ceil(tiles / 8) tiles for the wavefronts of an eighth of them.
+struct BackGrid {
+  int blocks, runs;
+};
+BackGrid back_grid(int tiles) {
+  int blocks = std::min(kBackBlocks, dec::xcd_grid(tiles, kInfWaves));
+  int per = blocks / 8 * kInfWaves * kBackTiles, eighth = (tiles + 7) / 8;
+  return {blocks, (eighth + per - 1) / per};
+}
+
 // The forward pass on the tile kernels after the scales: h3 and y (or, with
 // the errors e, eps in place of y) and c, each where given.
 void forward_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, const float *e, unsigned short *h3,
@@ -2296,12 +2320,13 @@ void loss_grad_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r,
   forward_tiles(nn, L, B, r, e, A.h3, e ? nn.eps.p : nn.y.p, nullptr, st);
   dim3 gv(dec::nblocks(n, TB), B);
   int tiles = tile_count(n, B);
-  int blocks = std::min(kBackBlocks, dec::xcd_grid(tiles, kInfWaves));
+  const auto [blocks, runs] = back_grid(tiles);
+  grow(nn.part, static_cast<size_t>(blocks) * NP);
   if (!e) {
     hipLaunchKernelGGL(k_loss, gv, dim3(TB), 0, st, n, B, L.a.width, L.a.col.p, L.a.val.p, nn.x.p, nn.y.p, L.D.p,
                        nullptr, nn.drho.p, nn.dpart.p);
     hipLaunchKernelGGL(k_head_back<false>, dim3(blocks), dim3(TB), 0, st, n, B, 0, L.at.width, L.at.col.p, L.at.val.p,
-                       nn.drho.p, nullptr, 1.0f, L.D.p, nn.x.p, A.h3, nn.dm.p, nn.part.p);
+                       nn.drho.p, nullptr, 1.0f, L.D.p, nn.x.p, A.h3, nn.dm.p, nn.part.p, runs);
   } else {
     dim3 gc(dec::nblocks(L.nc, TB), B);
     hipLaunchKernelGGL(k_bspmv, gc, dim3(TB), 0, st, L.nc, n, L.r.width, L.r.col.p, L.r.val.p, nn.eps.p, nn.crs.p);
@@ -2311,16 +2336,16 @@ void loss_grad_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r,
                        nn.crs.p);
     hipLaunchKernelGGL(k_head_back<true>, dim3(blocks), dim3(TB), 0, st, n, B, L.nc, L.rt.width, L.rt.col.p,
                        L.rt.val.p, nn.eps.p, nn.crs.p, 2.0f * L.dmean / (static_cast<float>(n) * B), L.D.p, nn.x.p,
-                       A.h3, nn.dm.p, nn.part.p);
+                       A.h3, nn.dm.p, nn.part.p, runs);
   }
   DEC_ELL_WIDTH_SWITCH(L.pt.width, if constexpr (W > 0) {
     hipLaunchKernelGGL((k_layer_back<W, true>), dim3(blocks), dim3(TB), 0, st, n, B, L.pt.col.p, L.pt.val.p,
                        static_cast<const unsigned short *>(nullptr), nn.dm.p, th + OWO, A.h2, th + OW3, A.dz,
-                       static_cast<const float *>(nullptr), static_cast<const float *>(nullptr), nn.part.p, OW3, OB2,
-                       OB3);
+                       static_cast<const float *>(nullptr), static_cast<const float *>(nullptr), nn.part.p, runs, OW3,
+                       OB2, OB3);
     hipLaunchKernelGGL((k_layer_back<W, false>), dim3(blocks), dim3(TB), 0, st, n, B, L.pt.col.p, L.pt.val.p, A.dz,
                        static_cast<const float2 *>(nullptr), static_cast<const float *>(nullptr), A.h1, th + OW2,
-                       static_cast<unsigned short *>(nullptr), nn.x.p, nn.px.p, nn.part.p, OW2, OB1, 0);
+                       static_cast<unsigned short *>(nullptr), nn.x.p, nn.px.p, nn.part.p, runs, OW2, OB1, 0);
   });
   hipLaunchKernelGGL(k_reduce_params, dim3((NP + 63) / 64 + 1), dim3(1024), 0, st, blocks, nn.part.p, nn.grad.p,
                      static_cast<int>(gv.x) * B, nn.dpart.p, 1.0 / (static_cast<double>(n) * B), loss_out);
