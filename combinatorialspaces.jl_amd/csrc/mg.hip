@@ -569,8 +569,10 @@ __global__ void k_perm_scatter(int n, const int *__restrict__ perm, const T *__r
 // pass adds Σ_c part[c * n + i] (c ascending) to u.  The fused coarse tail
 // uses the same two sums in the same order.
 // (16 columns where the coarse tail, whose threads hold a chunk's part of a row in
-// registers, can be the one that multiplies: its LDS ends at 1,792 beside 3,072 rows.
-// 64 above, for fewer partial sums.)
+// registers, can be the one that multiplies; 64 above, for fewer partial sums.  1,792 is
+// a choice: a dense level has a quarter of the rows above it in a refined mesh, so at most
+// 768 beside the tail's 3,072; 1,792 leaves room for hierarchies that coarsen less, and the
+// tail's LDS would hold 2,047.)
 __host__ __device__ inline int coarse_chunk(int n) { return n <= 1792 ? 16 : 64; }
 
 template <class T>
@@ -2210,11 +2212,12 @@ void build_panels(Level &L, const std::vector<int32_t> &color) {
 }
 
 // The rows of the coarse tail (see Tail) of a level that can be one: every row
-// with a diagonal, at most 7 other entries, and vectors that fit in 64 KiB of LDS.
-void build_tail(Level &L, const LevelDesc<double> &D) {
+// with a diagonal, at most 7 other entries, vectors that fit in 64 KiB of LDS, and
+// above the dense coarsest level its product in chunks of 16.
+void build_tail(Level &L, const LevelDesc<double> &D, bool above_dense) {
   const int n = L.n, S = std::max(L.width - 1, 1);
   if (n < 1 || n > kTailRows || L.width < 1 || L.width > 8 || L.ncolors > 15 || L.nc < 1 ||
-      coarse_chunk(L.nc) != 16 || tail_lds(n, L.nc, sizeof(double)) > 64 * 1024)
+      (above_dense && coarse_chunk(L.nc) != 16) || tail_lds(n, L.nc, sizeof(double)) > 64 * 1024)
     return;
   for (int r = 0; r < n; r++) {
     int diag = 0;
@@ -2580,7 +2583,7 @@ void finish_hierarchy(dec_mg_s &mg, const std::vector<dec::HostCsr> &As, std::ve
     mg.hdesc64 = d64;
     mg.hdesc32 = d32;
   }
-  for (int l = 0; l + 1 < nl; l++) build_tail(*mg.lv[l], mg.hdesc64[l]);
+  for (int l = 0; l + 1 < nl; l++) build_tail(*mg.lv[l], mg.hdesc64[l], l + 2 == nl);
   mg.part.alloc(4 * kCgBlocksMax);  // also the dot partials (kDotBlocks of them)
   mg.part2.alloc(4 * kCgBlocksMax);
   mg.scal.alloc(8);

@@ -15,7 +15,7 @@ CASES = [
     ((2, 1), (1,)), ((5, 2), (1, 3)), ((255, 64), (1,)), ((1023, 255), (1, 37)), ((1024, 257), (1, 37, 38)),
     ((1025, 500), (1, 41)), ((2048, 1100), (1, 2)), ((2049, 150), (1, 41, 42)), ((3000, 1500), (1,)),
     ((3000, 642), (1, 61, 62)), ((2500, 625), (1, 2, 61, 62)), ((2600, 650, 160, 40), (1, 51, 52)),
-    ((4001, 2000, 1000, 500), (1,)), ((9000, 1200, 300, 75), (1, 91)),
+    ((3000, 1900, 400), (1,)), ((4001, 2000, 1000, 500), (1,)), ((9000, 1200, 300, 75), (1, 91)),
 ]
 
 
