@@ -67,18 +67,6 @@ __device__ __forceinline__ void ast<unsigned short>(unsigned short *p, size_t i,
 template <>
 __device__ __forceinline__ void ast<float>(float *p, size_t i, float v) { p[i] = v; }
 
-__device__ __forceinline__ float ell_row(int n, int width, int r, const int *__restrict__ col,
-                                         const float *__restrict__ val, const float *__restrict__ x) {
-  float acc = 0.0f;
-  for (int k = 0; k < width; k++) {
-    size_t q = static_cast<size_t>(k) * n + r;
-    int c = col[q];
-    if (c < 0) break;
-    acc = acc + val[q] * x[c];
-  }
-  return acc;
-}
-
 // ---- forward ------------------------------------------------------------
 
 // Per-sample scale s_b = sqrt(mean r²): kScaleBlocks partial sums per sample
@@ -242,11 +230,11 @@ __global__ void k_dense_f32(int rows, const float *__restrict__ h, const float *
   out[row * H + col] = z > 0.0f ? z : 0.0f;
 }
 
-// y = alpha x + h3 wo + bo; c = (s / D) y, optionally u += c.
+// y = alpha x + h3 wo + bo; c = (s / D) y.
 template <class AT>
 __global__ void k_output(int n, const float *__restrict__ x, const AT *__restrict__ h3, const float *__restrict__ th,
                          const float *__restrict__ s, const float *__restrict__ D, float *__restrict__ y,
-                         float *__restrict__ c, float *__restrict__ u_add) {
+                         float *__restrict__ c) {
   int v = blockIdx.x * blockDim.x + threadIdx.x;
   int b = blockIdx.y;
   if (v >= n) return;
@@ -256,9 +244,7 @@ __global__ void k_output(int n, const float *__restrict__ x, const AT *__restric
   for (int j = 0; j < H; j++) hw = hw + ald(h3, o * H + j) * th[OWO + j];
   float yy = acc + hw + th[OBO];
   if (y) y[o] = yy;
-  float cc = (s[b] / D[v]) * yy;
-  if (c) c[o] = cc;
-  if (u_add) u_add[o] = u_add[o] + cc;
+  if (c) c[o] = (s[b] / D[v]) * yy;
 }
 
 // ---- inference: the smoother inside V-cycles -------------------------------
@@ -2182,13 +2168,12 @@ struct dec_nn_s {
   DBuf<float> th, grad, m1, m2;
   int adam_t = 0;
   // work buffers (grown on demand)
-  DBuf<float> x, px, y, c, s, drho, dg, part, r, eps, tmp, crs;
+  DBuf<float> x, px, y, c, s, drho, dg, part, eps, tmp, crs;
   DBuf<double> dpart, dloss, spart, rtmp;
   DBuf<float2> ix;                                 // inference: (x, P x)
   DBuf<unsigned short> ih1, ih2;                   // inference: layer-1 and layer-2 rows
   DBuf<unsigned char> h1, hm1, h2, hm2, h3, dz;  // activation storage (bf16 or f32)
   DBuf<float2> dm;                                 // (dy, signs of h3) per row
-  DBuf<int32_t> idx;
 };
 
 namespace {
@@ -2352,8 +2337,7 @@ void loss_grad_tiles(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r,
 }
 
 template <class AT>
-void forward_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, float *c_out, float *u_add,
-               hipStream_t st) {
+void forward_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, float *c_out, hipStream_t st) {
   int n = L.n;
   size_t rows = static_cast<size_t>(n) * B;
   Mode mode = mode_of<AT>(L);
@@ -2375,7 +2359,7 @@ void forward_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, float
   dense<AT>(R, A.h1, A.m1, th + OW2, th + OB2, A.h2, st);
   hipLaunchKernelGGL(k_spmm<AT>, gf, dim3(TB), 0, st, n, L.p.width, L.p.col.p, L.p.val.p, A.h2, A.m2);
   dense<AT>(R, A.h2, A.m2, th + OW3, th + OB3, A.h3, st);
-  hipLaunchKernelGGL(k_output<AT>, gv, dim3(TB), 0, st, n, nn.x.p, A.h3, th, nn.s.p, L.D.p, nn.y.p, c_out, u_add);
+  hipLaunchKernelGGL(k_output<AT>, gv, dim3(TB), 0, st, n, nn.x.p, A.h3, th, nn.s.p, L.D.p, nn.y.p, c_out);
 }
 
 // Loss (into *loss_out, device) and gradient (into nn.grad) of a batch of B
@@ -2389,7 +2373,7 @@ void loss_grad_t(dec_nn_s &nn, const dec::NnLevel &L, int B, const float *r, con
     loss_grad_tiles(nn, L, B, r, e, loss_out, st);
     return;
   }
-  forward_t<AT>(nn, L, B, r, nullptr, nullptr, st);
+  forward_t<AT>(nn, L, B, r, nullptr, st);
   int n = L.n;
   int R = n * B;
   Acts<AT> A = acts<AT>(nn);
@@ -2604,8 +2588,8 @@ int dec_nn_forward(dec_nn nn, int32_t level, int32_t nsamples, const float *r, f
   if (!nn || !r || !c || nsamples <= 0) fail(DEC_ERR_ARG, "dec_nn_forward: bad argument");
   const dec::NnLevel &L = level_of(*nn, level);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (precise) forward_t<float>(*nn, L, nsamples, r, c, nullptr, s);
-  else forward_t<unsigned short>(*nn, L, nsamples, r, c, nullptr, s);
+  if (precise) forward_t<float>(*nn, L, nsamples, r, c, s);
+  else forward_t<unsigned short>(*nn, L, nsamples, r, c, s);
   dec::check_launch("dec_nn_forward");
   DEC_CATCH
 }

@@ -95,17 +95,6 @@ __global__ void __launch_bounds__(256) k_sum_rows(int nb, const double *__restri
   if (threadIdx.x == 0) *out = sh[0];
 }
 
-// y[v] = (A x)[v]
-template <int W, class T>
-__global__ void k_spmv_rows(int n, int width, const int *__restrict__ col, const T *__restrict__ val,
-                            const int *__restrict__ rowid, const T *__restrict__ x, T *__restrict__ y,
-                            const int *__restrict__ done) {
-  if (done && *done) return;
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  y[rowid[p]] = dec_ell::row<W, T, T>(n, width, p, col, val, x);
-}
-
 // One colour of Gauss-Seidel: u[v] = (b[v] - Σ_{w≠v} A[v,w] u[w]) / A[v,v].
 template <int W, class T>
 __global__ void k_gs_color(int p0, int p1, int n, int width, const int *__restrict__ col,
@@ -1394,11 +1383,6 @@ __global__ void k_add_f2d(int n, const float *__restrict__ c, double *__restrict
   if (i < n) u[i] = u[i] + static_cast<double>(c[i]);
 }
 
-__global__ void k_f2d(int n, const float *__restrict__ c, double *__restrict__ z) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) z[i] = static_cast<double>(c[i]);
-}
-
 // ---------------------------------------------- V-cycle-preconditioned CG
 // Conjugate gradients on the finest level with one V-cycle (from a zero
 // start) as the preconditioner z = M r:
@@ -1979,8 +1963,6 @@ struct dec_mg_s {
   int fuse_from = -1;           // first level handled by the fused coarse kernel
   DBuf<LevelDesc<double>> desc64;
   DBuf<LevelDesc<float>> desc32;
-  std::vector<LevelDesc<double>> hdesc64;  // host copies (kernel arguments)
-  std::vector<LevelDesc<float>> hdesc32;
   bool use_fused = true;
   int fuse_rows = kFuseRowsDefault;
   // graph of one solve cycle or preconditioned-CG iteration (per variant)
@@ -2027,13 +2009,6 @@ struct dec_mg_s {
 namespace {
 
 inline dim3 G(long long n) { return dim3(dec::nblocks(n, kBlock)); }
-
-template <class T>
-const std::vector<LevelDesc<T>> &host_desc(const dec_mg_s &mg);
-template <>
-const std::vector<LevelDesc<double>> &host_desc<double>(const dec_mg_s &mg) { return mg.hdesc64; }
-template <>
-const std::vector<LevelDesc<float>> &host_desc<float>(const dec_mg_s &mg) { return mg.hdesc32; }
 
 template <class T>
 LevelVals<T> &vals(Level &L);
@@ -2580,10 +2555,8 @@ void finish_hierarchy(dec_mg_s &mg, const std::vector<dec::HostCsr> &As, std::ve
     }
     mg.desc64.upload(d64);
     mg.desc32.upload(d32);
-    mg.hdesc64 = d64;
-    mg.hdesc32 = d32;
+    for (int l = 0; l + 1 < nl; l++) build_tail(*mg.lv[l], d64[l], l + 2 == nl);
   }
-  for (int l = 0; l + 1 < nl; l++) build_tail(*mg.lv[l], mg.hdesc64[l], l + 2 == nl);
   mg.part.alloc(4 * kCgBlocksMax);  // also the dot partials (kDotBlocks of them)
   mg.part2.alloc(4 * kCgBlocksMax);
   mg.scal.alloc(8);
@@ -2989,7 +2962,6 @@ void coarse_solve(dec_mg_s &mg, Level &L, const T *b, T *u, hipStream_t s) {
   (void)mg;
 }
 
-// _multigrid_μ_cycle (Multigrid.jl:857-872).
 // The coarse tail's launch at level l, on the way down (C's solution, or above
 // the level before the last C's right-hand side, from b and u; the smoothed u goes to
 // the level's r) or up.
@@ -3029,6 +3001,7 @@ void tail_launch(dec_mg_s &mg, int l, const T *b, T *u, bool u_zero, bool up, hi
   }
 }
 
+// _multigrid_μ_cycle (Multigrid.jl:857-872).
 template <class T>
 void mu_cycle(dec_mg_s &mg, int lvl, T *u, const T *b, int mu, bool u_zero, hipStream_t s) {
   int nl = static_cast<int>(mg.lv.size());
