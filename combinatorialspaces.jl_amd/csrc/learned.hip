@@ -1500,19 +1500,24 @@ __global__ void __launch_bounds__(TB, 3)
   }
   int wt, wend, step;
   wave_tiles(B * T, wt, wend, step);
+  wt = __builtin_amdgcn_readfirstlane(wt);  // (the same over the wavefront: its tile's arithmetic in scalar registers)
   // One 16-row group at a time, four to a tile: the rows pass through 8.7 KB of
-  // LDS a wavefront, so that three workgroups fit in a CU by their registers (64
-  // rows at once: 17 KB, two workgroups), and the groups are not unrolled, which
+  // LDS a wavefront, so that three workgroups fit in a CU (64 rows at once: 17 KB,
+  // two workgroups), and the groups are not unrolled, which
   // keeps their addresses out of registers.  16 x 40,962 rows, HEAD and not: 63
   // and 70 µs with 64 rows at once and columns read entry by entry, 56 and
   // 38 so; with the next group's gathers issued ahead of the products, two
   // workgroups a CU, 58 and 41; held to four, with spills, 61 and 42.
   int c[W];
   float pv[W];
-  // the sums in double: wave w holds dW's registers k = w, w + 4, ... (see v below), thread t < kCols the t-th of
+  // the sums in double: wave w holds dW's registers k = w, w + 4, ... (see v below), in LDS, since rows of 8 slots
+  // leave no registers for them (64 x 41,000 such rows: 870 µs a gradient against 930); thread t < kCols the t-th of
   // the columns' sums: the bias below, then dz's own (HEAD) or W1's
   constexpr int kCols = HEAD ? 2 * H : 3 * H;
-  double dW[32 / kInfWaves] = {}, dcol = 0.0;
+  __shared__ double dW_s[32 / kInfWaves][TB];
+  double dcol = 0.0;
+#pragma unroll
+  for (int j = 0; j < 32 / kInfWaves; j++) dW_s[j][threadIdx.x] = 0.0;
 #pragma unroll 1
   for (int run = 0; run < runs; run++) {
     float4_t aO[2][2], aN[2][2];  // dW tiles: features 16 ft.., columns 16 jt..
@@ -1697,9 +1702,12 @@ __global__ void __launch_bounds__(TB, 3)
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 32 / kInfWaves; j++)
+    for (int j = 0; j < 32 / kInfWaves; j++) {
+      double t = dW_s[j][tid];
 #pragma unroll
-      for (int q = 0; q < kInfWaves; q++) dW[j] = dW[j] + static_cast<double>(lds[(q * 32 + kInfWaves * j + w) * 64 + l]);
+      for (int q = 0; q < kInfWaves; q++) t = t + static_cast<double>(lds[(q * 32 + kInfWaves * j + w) * 64 + l]);
+      dW_s[j][tid] = t;
+    }
     if (tid < kCols) {
 #pragma unroll
       for (int q = 0; q < kInfWaves; q++) dcol = dcol + static_cast<double>(cols[q * kCols + tid]);
@@ -1710,7 +1718,7 @@ __global__ void __launch_bounds__(TB, 3)
 #pragma unroll
   for (int j = 0; j < 32 / kInfWaves; j++) {
     int k = kInfWaves * j + wv, f = H * (k >> 4) + 16 * ((k >> 3) & 1) + 4 * lg + (k & 3), col = 16 * ((k >> 2) & 1) + li;
-    out[ow + f * H + col] = static_cast<float>(dW[j]);
+    out[ow + f * H + col] = static_cast<float>(dW_s[j][threadIdx.x]);
   }
   if (threadIdx.x < kCols) {
     int t = threadIdx.x, second = HEAD ? ob_self : OW1;
