@@ -1196,7 +1196,7 @@ __global__ void k_hp_grad(int n, float scale, const float *__restrict__ eh, cons
 //
 // What bounds them: the h and dz rows read and written (0.46 GB at 16 x 40,962
 // rows, about 90 µs of HBM time) and the gathers' dependent loads.  Measured at
-// that size, loss and gradient of the error loss: 271 µs, against 2,020 µs with
+// that size, loss and gradient of the error loss: 273 µs, against 2,020 µs with
 // one kernel per operation (dg in FP32, two launches per reduction), the
 // gradient as far from its value in 64 bits as before (4.1e-3 of its norm).
 
@@ -1505,7 +1505,7 @@ __global__ void __launch_bounds__(TB, 3)
   // LDS a wavefront, so that three workgroups fit in a CU (64 rows at once: 17 KB,
   // two workgroups), and the groups are not unrolled, which
   // keeps their addresses out of registers.  16 x 40,962 rows, HEAD and not: 63
-  // and 70 µs with 64 rows at once and columns read entry by entry, 56 and
+  // and 70 µs with 64 rows at once and columns read entry by entry, 54 and
   // 38 so; with the next group's gathers issued ahead of the products, two
   // workgroups a CU, 58 and 41; held to four, with spills, 61 and 42.
   int c[W];
