@@ -399,9 +399,8 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int m = 0; m < 2; m++) {
     int i = t + m * nt;
-    if (i < P.hs) x[P.B + i] = ZERO ? static_cast<T>(0) : hv[m];
+    if (i <= P.hs) x[P.B + i] = ZERO || i == P.hs ? static_cast<T>(0) : hv[m];  // the halo, then the zero
   }
-  if (t == 0) x[P.B + P.hs] = static_cast<T>(0);
   __syncthreads();
   int color[R], row[R];
 #pragma unroll
@@ -880,7 +879,7 @@ __global__ void __launch_bounds__(kBlock)
       // too much cancelled: the sum itself, by every workgroup in the same order (a
       // pass over r and Ap by each, on the rare step that cuts ‖r‖ a thousandfold)
       double g[1] = {0.0};
-#pragma unroll 4
+#pragma unroll 1
       for (int i = threadIdx.x; i < n; i += kBlock) {
         double v = next_r(r0[i], a, q0[i]);
         g[0] = g[0] + v * v;
@@ -2132,7 +2131,7 @@ void build_panels(Level &L, const std::vector<int32_t> &color) {
   const dec::HostCsr &A = L.A;
   const int n = L.n, B = L.panel_b, nb = L.nblk, S = L.width - 1;
   if (L.width < 2 || L.width > 8 || L.ncolors > 16) return;
-  const int most = 2 * panel_threads(B);
+  const int most = 2 * panel_threads(B) - 1;  // (and the zero behind the halo)
   std::vector<int32_t> order(n), stamp(n, -1), halo, count(nb), first(nb + 1, 0);
   int hs = 1;
   for (int k = 0; k < nb; k++) {
